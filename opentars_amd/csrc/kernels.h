@@ -71,6 +71,11 @@ __device__ __forceinline__ int xcd_block(int x, int n) {
   return r * per + min(r, rem) + k;
 }
 
+// Row m of fp32 rows at a byte stride.
+__device__ __forceinline__ const float* frow_f32(const void* base, int64_t ld, int m) {
+  return reinterpret_cast<const float*>(static_cast<const char*>(base) + m * ld);
+}
+
 // Kernel-argument preloading (the library is built with -amdgpu-kernarg-preload-count): gfx950
 // places the leading scalar kernel arguments in SGPRs at wave launch, so a kernel whose first
 // loads need only those issues them without a kernel-argument round trip. Kernels on the latency
@@ -357,6 +362,9 @@ struct EmbedArgs {
 };
 hipError_t launch_embed_rows(const EmbedArgs& a, hipStream_t s);
 hipError_t launch_attention(const AttnArgs& a, hipStream_t s);
+// Prompt rows (attn_rows.hip): 16 query rows of a head per workgroup; the arguments of launch_attention
+// (no scratch, no norm + RoPE prologue).
+hipError_t launch_attention_rows(const AttnArgs& a, hipStream_t s);
 
 hipError_t launch_row(const RowArgs& a, hipStream_t s);
 // An ELT ADD (dense fp32 rows, fp32 output, no activation) and the LayerNorm / RMSNorm / L2Norm of

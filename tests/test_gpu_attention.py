@@ -100,6 +100,49 @@ def test_attention_with_values_the_flushes_change(heads, kv_heads, hd, M, t0, v_
     run_case(heads, kv_heads, hd, M, t0, v_fp16, OUT_FP32, specials=True)
 
 
+# prompt rows (16 query rows per workgroup): one row of a tile, whole and partial tiles, every head size
+# and V format, both sides of the key count past which a tile holds 8 rows (2544 keys)
+PROMPT_CASES = [
+    (16, 8, 128, 5, 60, False, OUT_INT8, False),
+    (2, 1, 64, 16, 0, False, OUT_FP32, False),
+    (8, 4, 64, 17, 3, True, OUT_BF16, False),
+    (3, 3, 128, 33, 100, False, OUT_FP32, True),
+    (2, 1, 256, 40, 30, True, OUT_FP32, True),
+    (8, 8, 256, 18, 7, False, OUT_FP32, True),
+    (2, 2, 64, 20, 2520, False, OUT_FP32, False),
+    (1, 1, 64, 9, 2540, False, OUT_FP32, True),
+    (1, 1, 128, 23, 4050, True, OUT_FP32, False),
+]
+
+
+@pytest.mark.parametrize("heads,kv_heads,hd,M,t0,v_fp16,out,specials", PROMPT_CASES)
+def test_attention_of_prompt_rows(heads, kv_heads, hd, M, t0, v_fp16, out, specials):
+    run_case(heads, kv_heads, hd, M, t0, v_fp16, out, specials)
+
+
+@pytest.mark.parametrize("v_fp16", [False, True])
+def test_masked_keys_of_prompt_rows_that_change_a_sum(v_fp16):
+    """Keys no row of a tile sees still take part in P V with probability +0: an infinite V element
+    there makes NaN, and a sum that was flushed to -0 becomes +0 (or stays -0, by the V signs)."""
+    M, nk, hd, causal_k = 40, 160, 64, 20
+    rng = np.random.default_rng(5)
+    q, kc, vv = (rng.normal(0, 0.5, s).astype(f32) for s in ((M, hd), (nk, hd), (nk, hd)))
+    kc[1] = kc[0]
+    vv[nk - 1, 7] = np.inf                              # masked for every row
+    vv[causal_k + 30, 9] = np.nan                       # masked for the first rows only
+    if not v_fp16:                                      # p0 v0 + p1 v1 = -2^-126 p, flushed to -0
+        vv[0, 3:5], vv[1, 3:5] = f32(2.0 ** -103) * f32(1 - 2.0 ** -23), -f32(2.0 ** -103)
+        vv[2:causal_k + M, 3:5] = -0.0
+        vv[causal_k + M:, 3], vv[causal_k + M:, 4] = 1.0, -1.0
+    vdev = vv.astype(np.float16).view(np.uint16) if v_fp16 else vv
+    vval = F.from_fp16_bits(vdev) if v_fp16 else vv
+    got = ops.attention(q, kc, vdev, 1, 1, causal_k=causal_k, v_fp16=v_fp16)
+    want = oracle_attention(q, kc, vval, 1, 1, hd, causal_k, OUT_FP32, None)[0]
+    if not v_fp16:
+        assert np.all(bits(want[:, 3]) == 0) and np.all(bits(want[:, 4]) == 0x80000000)
+    assert np.array_equal(bits(got), bits(want))
+
+
 def test_attention_twice_in_a_row_and_without_the_shared_rows():
     """Two calls on one stream share the device scratch: the second (fewer keys, other heads)
     must not see the first's scores; sc / pr left out."""
