@@ -24,11 +24,24 @@
 //     levels join the four e of a block, the last two the blocks: registers only, no lane exchange.
 //  2. softmax, 16 lanes per row: the maximum, then exp and the 16-lane sum in one pass, then the
 //     products with the reciprocal.
-//  3. P V: wave w takes output columns 64 w .. + 63 (block b columns 16 b .. + 15), keys in order.
-//     Keys past the last one any row of the tile may see are left out of both products: their
-//     probabilities are +0, and acc + (+-0) = acc unless acc is -0 or the V element is infinite or
-//     NaN; a scan of those V elements and of the sums decides, and the keys run if need be.
+//  3. P V: a wave takes RW rows x 64 columns, keys in order, on v_mfma_f32_4x4x1_16b_f32 (4 rows x 64
+//     columns of products; lane = column). V rows come by buffer loads two 16-key blocks ahead, the first
+//     before the softmax. Keys past the last one any row of the tile may see are left out of both
+//     products: their probabilities are +0, and acc + (+-0) = acc unless acc is -0 or the V element is
+//     infinite or NaN; a scan of those V elements and of the sums decides, and the keys run if need be.
+//
+// Measured on MI355X. f32 MFMA and vector adds do not overlap there: per 64 products and sums 4.5 - 4.8
+// cycles of a SIMD with two or more waves (a product by v_mul costs the same 2.4 cycles as its share of
+// an MFMA, but needs its operands spread over the lanes), 7.5 - 8 with one wave, which issues a vector
+// instruction every 4.9 cycles at best. So the split aims at two waves per SIMD: 8 rows per P V wave (4
+// waves at head size 128) when the grid gives more than a workgroup per CU, else 4 rows (8 waves):
+// 128 rows of 8 heads over 512 keys 50 -> 45 us with 4; 512 rows of 16 heads, causal, 55 us with 8 and
+// 68 us with 4. Steps from the first form (64 columns x 16 rows per P V wave on the 16 x 16 x 1 MFMA,
+// 110 us there): 8 rows per wave 75, straight-line softmax 68, buffer loads with scalar row offsets 61
+// (64-bit lane addresses cost a quarter-rate add per load), probabilities always from LDS 55.
+// One workgroup per head, row by row, took 11.7 ms.
 #include <mutex>
+#include <type_traits>
 
 #include "kernels.h"
 #include "row_sums.h"
@@ -37,8 +50,12 @@ namespace tars {
 namespace {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int kTile = 16;  // query rows per workgroup, keys per scores tile
+constexpr int kKeys = 16;  // keys per block of P V
+constexpr int kAhead = 2;  // blocks of V rows in flight
+constexpr size_t kLds = 163840;  // LDS of a CU
 
 // fp32 subnormals kept / flushed (MODE bits 4-5) from here on. The values an instruction of a region
 // takes or gives pass through tie() inside it: the compiler keeps volatile statements in order, so
@@ -70,12 +87,14 @@ __device__ __forceinline__ v16f products(float a, float b, const v16f& neg0) {
   return d;
 }
 
-template <int HD, bool VHALF>
-__global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_rows_kernel(AttnArgs a, int tr, int lds_row, int tiles) {
-  constexpr int U = HD / 16, NWV = HD / 64;
+// RW: query rows per P V wave (4 or 8); the workgroup has 16 / RW * HD / 64 waves
+template <int HD, bool VHALF, int RW>
+__global__ __launch_bounds__(64 * (16 / RW) * (HD / 64), 2) void attn_rows_kernel(AttnArgs a, int tr, int lds_row,
+                                                                                   int tiles) {
+  constexpr int U = HD / 16, nw = 16 / RW * (HD / 64);
   extern __shared__ __align__(16) float sp[];  // [tr][lds_row]
   const int t = threadIdx.x, lane = t & 63, l = lane & 15, lg = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), nw = blockDim.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   // Workgroups are dealt round-robin over the 8 XCDs: with the heads a multiple of 8 each XCD gets
   // heads / 8 consecutive ones, so a K / V head is read through one L2. The last rows first: they see
   // the most keys.
@@ -161,131 +180,189 @@ __global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_rows_kernel(AttnA
       }
     }
   }
+  // ---- P V operands: RW rows x 64 columns per wave
+  constexpr int NC = HD / 64, ES = VHALF ? 2 : 4, H4 = RW / 4;
+  const int cg = wave % NC, r0 = wave / NC * RW;
+  const int pad = (limit + 15) / 16 * 16;  // P V runs over whole blocks of 16 keys
+  const char* vcol = static_cast<const char*>(a.v[h]) + 64 * ES * cg;
+  // V elements (as stored) of keys j0 .. j0 + kKeys - 1 (j0 < nk); past the matrix the last row's again
+  struct Keys {
+    uint32_t v[kKeys];
+  };
+  const int ldv = static_cast<int>(a.ldv);
+  auto load = [&](Keys& o, int j0) __attribute__((always_inline)) {
+    // buffer loads: the block's base in the resource, the row's offset scalar, the lane's column in a VGPR
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(vcol) + static_cast<int64_t>(j0) * a.ldv, 0,
+                                                        -1, 0x00027000);
+    const int left = nk - 1 - j0;
+#pragma unroll
+    for (int i = 0; i < kKeys; ++i) {
+      const int row = min(i, left) * ldv;
+      if constexpr (VHALF) o.v[i] = __builtin_amdgcn_raw_buffer_load_b16(rsrc, ES * lane, row, 0);
+      else o.v[i] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, ES * lane, row, 0);
+    }
+  };
+  // the first blocks' V rows, in flight while the softmax runs
+  Keys vq[kAhead];
+#pragma unroll
+  for (int i = 0; i < kAhead; ++i) load(vq[i], min(i * kKeys, nk - 1));
   __syncthreads();
 
   // ---- 2. softmax: 16 lanes per row
-  const int pad = (limit + 15) / 16 * 16;  // P V runs over whole blocks of 16 keys
-  for (int r = t >> 4; r < tr; r += blockDim.x >> 4) {
+  for (int r = t >> 4; r < tr; r += 4 * nw) {
     float* s = sp + r * lds_row;
     const int m = m0 + min(r, rows - 1);
     const int V = a.causal_k > 0 ? min(nk, a.causal_k + m) : nk;
+    // the lane's n elements l, l + 16, ... of the row, eight at a time (their chains of steps side by side)
+    const int n = pad >> 4;
+    auto each = [&](auto&& f) {
+      int i = 0;
+      for (; i + 8 <= n; i += 8) f(i, std::integral_constant<int, 8>{});
+      for (; i < n; ++i) f(i, std::integral_constant<int, 1>{});
+    };
     uint32_t key = 0;
-    for (int j0 = l; j0 < V; j0 += 128) {
-      float x[8];
+    each([&](int i0, auto size) {
+      constexpr int B = decltype(size)::value;
+      float x[B];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) x[i] = s[min(j0 + 16 * i, V - 1)];  // a repeat changes no maximum
+      for (int i = 0; i < B; ++i) x[i] = s[l + 16 * (i0 + i)];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) key = max(key, is_nan(x[i]) ? 0xFFFFFFFFu : fmax_key(x[i]));
-    }
+      for (int i = 0; i < B; ++i) {
+        const uint32_t k = is_nan(x[i]) ? 0xFFFFFFFFu : fmax_key(x[i]);
+        key = l + 16 * (i0 + i) < V ? max(key, k) : key;
+      }
+    });
     key = static_cast<uint32_t>(group_reduce<16>(static_cast<int>(key), OpMaxU{}));
     const float nmx = fneg(key == 0xFFFFFFFFu ? ffrom(kCanonNaN) : fmax_from_key(key));
     // exp values are 0, normal, infinite or NaN, so their plain sums are the contract's
     float acc = 0.0f;
-    for (int j0 = l; j0 < pad; j0 += 64) {
-      float x[4];
+    each([&](int i0, auto size) {
+      constexpr int B = decltype(size)::value;
+      float x[B];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) x[i] = s[min(j0 + 16 * i, pad - 1)];
+      for (int i = 0; i < B; ++i) x[i] = s[l + 16 * (i0 + i)];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int j = j0 + 16 * i;
-        x[i] = j < V ? exp_f(fadd(x[i], nmx)) : 0.0f;
-        acc = __fadd_rn(acc, x[i]);
-        if (j < pad) s[j] = x[i];
+      for (int i = 0; i < B; ++i) {
+        const float e = exp_f(fadd(x[i], nmx));
+        x[i] = l + 16 * (i0 + i) < V ? e : 0.0f;
       }
-    }
+#pragma unroll
+      for (int i = 0; i < B; ++i) acc = __fadd_rn(acc, x[i]);
+#pragma unroll
+      for (int i = 0; i < B; ++i) s[l + 16 * (i0 + i)] = x[i];
+    });
     const float inv = recip_f(fold16(acc));
     const float zero = fmul(0.0f, inv);  // a masked probability: +0 (NaN when the row's sum is)
     float* prow = last && a.pr && r < rows
                       ? reinterpret_cast<float*>(reinterpret_cast<char*>(a.pr) + (m0 + r) * a.ldpr) : nullptr;
-    for (int j0 = l; j0 < pad; j0 += 64) {
-      float x[4];
+    each([&](int i0, auto size) {
+      constexpr int B = decltype(size)::value;
+      float x[B];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) x[i] = s[min(j0 + 16 * i, pad - 1)];
+      for (int i = 0; i < B; ++i) x[i] = s[l + 16 * (i0 + i)];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int j = j0 + 16 * i;
+      for (int i = 0; i < B; ++i) {
+        const int j = l + 16 * (i0 + i);
         const float p = fmul(x[i], inv);
         // past the matrix: -0, whose product with the +0 standing in for V leaves every sum as it is
-        if (j < pad) s[j] = j < nk ? p : -0.0f;
-        if (prow && j < min(pad, nk)) prow[j] = p;
+        s[j] = j < nk ? p : -0.0f;
+        if (prow && j < nk) prow[j] = p;
       }
-    }
+    });
     if (prow)
       for (int j = pad + l; j < nk; j += 16) prow[j] = zero;
   }
   __syncthreads();
 
-  // ---- 3. P V: 64 columns per wave
-  if (wave >= NWV) return;
-  constexpr int ES = VHALF ? 2 : 4;
-  const char* vcol = static_cast<const char*>(a.v[h]) + 64 * ES * wave;
-  const float* prow = sp + min(l, tr - 1) * lds_row;
-  struct Block {
-    uint32_t v[16];  // V elements as stored
-    float4 p[4];
-  };
-  auto load = [&](Block& o, int j0, bool probs) {
+  // ---- 3. P V
+  if (r0 >= rows) return;
+  // MFMA h (h < H4) takes rows r0 + 4 h .. + 3; its lane's operand row (a row past tr is clamped, unstored)
+  const float* prow[H4];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const char* p = vcol + static_cast<int64_t>(min(j0 + i, nk - 1)) * a.ldv + ES * lane;
-      if constexpr (VHALF) o.v[i] = *reinterpret_cast<const uint16_t*>(p);
-      else o.v[i] = *reinterpret_cast<const uint32_t*>(p);
-    }
+  for (int i = 0; i < H4; ++i) prow[i] = sp + min(r0 + 4 * i + (lane & 3), tr - 1) * lds_row;
+  v4f acc[H4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (probs) o.p[i] = *reinterpret_cast<const float4*>(prow + j0 + 4 * i);
-      else  // masked keys: probability +0 (-0 past the matrix)
-        o.p[i] = make_float4(j0 + 4 * i < nk ? 0.0f : -0.0f, j0 + 4 * i + 1 < nk ? 0.0f : -0.0f,
-                             j0 + 4 * i + 2 < nk ? 0.0f : -0.0f, j0 + 4 * i + 3 < nk ? 0.0f : -0.0f);
-    }
-  };
-  v16f acc = splat(0.0f);
-  // keys [j0, j1) (multiples of 16), the next block's V rows and probabilities loaded during a block's steps
-  auto chains = [&](int j0, int j1, bool probs) {
-    Block nxt;
-    load(nxt, j0, probs);
-    for (int j = j0; j < j1; j += 16) {
-      float v[16], p[16];
+  for (int i = 0; i < H4; ++i) acc[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  const v4f n0 = {-0.0f, -0.0f, -0.0f, -0.0f};
+  // kKeys keys from j on: their V rows in o (refilled with the block kAhead on when that is before j1), their
+  // probabilities from LDS. Four keys' products are formed while the four before are added.
+  auto block = [&](Keys& o, int j, int j1) __attribute__((always_inline)) {
+      float v[kKeys];
+      float4 p[H4][kKeys / 4];
+#pragma unroll
+      for (int i = 0; i < H4; ++i)
+#pragma unroll
+        for (int c = 0; c < kKeys / 4; ++c)
+          p[i][c] = *reinterpret_cast<const float4*>(prow[i] + j + 4 * c);
       flush_denorms();
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        v[i] = VHALF ? fp16_to_f32_keep_nan(nxt.v[i]) : ffrom(nxt.v[i]);
+      for (int i = 0; i < kKeys; ++i) {
+        v[i] = VHALF ? fp16_to_f32_keep_nan(o.v[i]) : ffrom(o.v[i]);
         if constexpr (!VHALF) flush_in_place(v[i]);
       }
-      if (j + 16 > nk) {
+      if (j + kKeys > nk) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = j + i < nk ? v[i] : 0.0f;
+        for (int i = 0; i < kKeys; ++i) v[i] = j + i < nk ? v[i] : 0.0f;
       }
+      if (j + kAhead * kKeys < j1) load(o, j + kAhead * kKeys);
+      auto quad = [&](v4f (&d)[4][H4], int c) __attribute__((always_inline)) {
+        keep_denorms();
 #pragma unroll
-      for (int i = 0; i < 4; ++i) p[4 * i] = nxt.p[i].x, p[4 * i + 1] = nxt.p[i].y, p[4 * i + 2] = nxt.p[i].z, p[4 * i + 3] = nxt.p[i].w;
-      if (j + 16 < j1) load(nxt, j + 16, probs);
-      v16f d = products(p[0], v[0], neg0);
+        for (int k = 0; k < 4; ++k) {
+          tie(v[4 * c + k]);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        v16f dn;
-        if (i + 1 < 16) dn = products(p[i + 1], v[i + 1], neg0);
-        tie(d);
-        acc = acc + d;
-        tie(acc);
-        if (i + 1 < 16) d = dn;
+          for (int i = 0; i < H4; ++i) {
+            const float4 q = p[i][c];
+            d[k][i] = __builtin_amdgcn_mfma_f32_4x4x1f32(k == 0 ? q.x : k == 1 ? q.y : k == 2 ? q.z : q.w, v[4 * c + k], n0,
+                                                         0, 0, 0);
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int i = 0; i < H4; ++i) tie(d[k][i]);
+        flush_denorms();
+      };
+      v4f d[2][4][H4];
+      quad(d[0], 0);
+#pragma unroll
+      for (int c = 0; c < kKeys / 4; ++c) {
+        if (c + 1 < kKeys / 4) quad(d[(c + 1) & 1], c + 1);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+#pragma unroll
+          for (int i = 0; i < H4; ++i) {
+            tie(d[c & 1][k][i]);
+            acc[i] = acc[i] + d[c & 1][k][i];
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < H4; ++i) tie(acc[i]);
       }
+  };
+  // the keys some row sees; then, if they can change a sum (see the file notes), the masked ones
+  for (int j0 = 0, j1 = pad;; j0 = pad, j1 = (nk + kKeys - 1) / kKeys * kKeys) {
+    for (int j = j0; j < j1; j += kAhead * kKeys) {
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i)
+        if (j + i * kKeys < j1) block(vq[i], j + i * kKeys, j1);
     }
     keep_denorms();
-  };
-  chains(0, pad, true);
-  if (pad < nk) {  // masked keys of every row (see the file notes)
+    if (j1 >= nk) break;
     bool need = false;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float x = acc[i];
-      need |= fbits(x) == kSign;
-    }
+    for (int i = 0; i < H4; ++i)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float x = acc[i][v];
+        need |= fbits(x) == kSign;
+      }
     constexpr int LPR = 64 * ES / 16;  // lanes per 64-column row piece
-    for (int j0 = pad + lane / LPR; j0 < nk; j0 += 4 * (64 / LPR)) {
+    for (int js = pad + lane / LPR; js < nk; js += 4 * (64 / LPR)) {
       uint4 w[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        w[i] = *reinterpret_cast<const uint4*>(vcol + static_cast<int64_t>(min(j0 + i * (64 / LPR), nk - 1)) * a.ldv +
+        w[i] = *reinterpret_cast<const uint4*>(vcol + static_cast<int64_t>(min(js + i * (64 / LPR), nk - 1)) * a.ldv +
                                                16 * (lane % LPR));
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -297,22 +374,28 @@ __global__ __launch_bounds__(256, HD == 256 ? 1 : 2) void attn_rows_kernel(AttnA
         }
       }
     }
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(need) != 0, 0)) chains(pad, (nk + 15) / 16 * 16, false);
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(need) == 0, 1)) break;
+    // their probabilities into this wave's rows (the waves of a row write the same values): +0, -0 past the matrix
+    for (int r = r0; r < min(r0 + RW, tr); ++r)
+      for (int j = pad + lane; j < (nk + kKeys - 1) / kKeys * kKeys; j += 64) sp[r * lds_row + j] = j < nk ? 0.0f : -0.0f;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) load(vq[i], min(pad + i * kKeys, nk - 1));
   }
 #pragma unroll
-  for (int blk = 0; blk < 4; ++blk)
+  for (int i = 0; i < H4; ++i)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const int r = 4 * lg + v;
-      const float y = acc[4 * blk + v];
-      if (r < rows) store_out(a.att[h], (m0 + r) * a.ldatt, 64 * wave + 16 * blk + l, a.out, chain_end(y), a.out_scale);
+      const int r = r0 + 4 * i + v;
+      const float y = acc[i][v];
+      if (r < rows) store_out(a.att[h], (m0 + r) * a.ldatt, 64 * cg + lane, a.out, chain_end(y), a.out_scale);
     }
 }
 
 // More than 64 KiB of dynamic LDS is asked for once per device and instance.
-template <int HD, bool VHALF>
-hipError_t go(const AttnArgs& a, hipStream_t s) {
-  constexpr size_t kLds = 163840;
+template <int HD, bool VHALF, int RW>
+hipError_t go(const AttnArgs& a, int tr, int lds_row, hipStream_t s) {
   static std::mutex mu;
   static bool ready[64] = {};
   int dev = -1;
@@ -321,31 +404,34 @@ hipError_t go(const AttnArgs& a, hipStream_t s) {
   {
     std::lock_guard<std::mutex> lock(mu);
     if (!ready[dev]) {
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attn_rows_kernel<HD, VHALF>),
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attn_rows_kernel<HD, VHALF, RW>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
       if (e != hipSuccess) return e;
       ready[dev] = true;
     }
   }
-  // row pitch 4 * odd: an MFMA operand read (16 rows x 16 bytes) and a scores store touch every
-  // bank once; 16 rows per workgroup while they fit, else 8
+  const int tiles = (a.M + tr - 1) / tr;
+  hipLaunchKernelGGL((attn_rows_kernel<HD, VHALF, RW>), dim3(static_cast<unsigned>(tiles) * a.heads),
+                     dim3(64 * (16 / RW) * (HD / 64)), static_cast<size_t>(4) * tr * lds_row, s, a, tr, lds_row, tiles);
+  return hipGetLastError();
+}
+
+template <bool VHALF>
+hipError_t rows(const AttnArgs& a, hipStream_t s) {
+  // row pitch 4 * odd: an MFMA operand read (16-byte pieces of several rows) and a scores store touch
+  // every bank once; 16 rows per workgroup while they fit, else 8
   const int lds_row = (a.nk + 15) / 16 * 16 + 4;
   const int tr = static_cast<size_t>(64) * lds_row <= kLds ? 16 : 8;
-  const size_t lds = static_cast<size_t>(4) * tr * lds_row;
-  const int tiles = (a.M + tr - 1) / tr;
-  // 4 waves (a wave per SIMD) where LDS leaves at most two workgroups per CU, else the P V waves alone
-  const int nw = kLds / lds <= 2 ? 4 : (HD / 64 > 2 ? HD / 64 : 2);
-  hipLaunchKernelGGL((attn_rows_kernel<HD, VHALF>), dim3(static_cast<unsigned>(tiles) * a.heads), dim3(64 * nw), lds, s, a, tr,
-                     lds_row, tiles);
-  return hipGetLastError();
+  if (a.hd == 64) return go<64, VHALF, 4>(a, tr, lds_row, s);
+  if (a.hd == 256) return go<256, VHALF, 8>(a, tr, lds_row, s);
+  const bool few = static_cast<int64_t>((a.M + tr - 1) / tr) * a.heads <= 256;
+  return few ? go<128, VHALF, 4>(a, tr, lds_row, s) : go<128, VHALF, 8>(a, tr, lds_row, s);
 }
 
 }  // namespace
 
 hipError_t launch_attention_rows(const AttnArgs& a, hipStream_t s) {
-  if (a.hd == 64) return a.v_fp16 ? go<64, true>(a, s) : go<64, false>(a, s);
-  if (a.hd == 128) return a.v_fp16 ? go<128, true>(a, s) : go<128, false>(a, s);
-  return a.v_fp16 ? go<256, true>(a, s) : go<256, false>(a, s);
+  return a.v_fp16 ? rows<true>(a, s) : rows<false>(a, s);
 }
 
 }  // namespace tars

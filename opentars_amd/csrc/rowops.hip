@@ -1387,8 +1387,8 @@ hipError_t launch_attention(const AttnArgs& in, hipStream_t s) {
   }
   const AttnArgs& a = in;
   // several rows the split form does not take: 16 rows per workgroup (512 rows of 16 heads over 512
-  // keys 11.7 -> 0.11 ms against one workgroup per head)
-  if (a.M >= 2) return launch_attention_rows(a, s);
+  // keys 11.7 ms -> 55 us against one workgroup per head); its V loads offset 16 rows in 32 bits
+  if (a.M >= 2 && a.ldv < (int64_t{1} << 27)) return launch_attention_rows(a, s);
   if (a.hd == 64) {
     if (a.v_fp16) hipLaunchKernelGGL((attn_kernel<64, true>), grid, block, 0, s, a);
     else hipLaunchKernelGGL((attn_kernel<64, false>), grid, block, 0, s, a);
