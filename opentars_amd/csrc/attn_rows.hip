@@ -129,8 +129,12 @@ __global__ __launch_bounds__(64 * (16 / RW) * (HD / 64), 2) void attn_rows_kerne
       for (int u = 0; u < U; ++u) kn[u] = *reinterpret_cast<const float4*>(kr + 16 * u);
     };
     const int nt = (score_keys + kTile - 1) / kTile;
-    if (wave < nt) load(wave);
+    // the next tile's K rows arrive during a tile's chains, but at head size 256, whose registers two tiles
+    // would not fit
+    constexpr bool kPrefetch = HD <= 128;
+    if (kPrefetch && wave < nt) load(wave);
     for (int kt = wave; kt < nt; kt += nw) {
+      if (!kPrefetch) load(kt);
       float k[4][U];
       flush_denorms();
 #pragma unroll
@@ -142,7 +146,7 @@ __global__ __launch_bounds__(64 * (16 / RW) * (HD / 64), 2) void attn_rows_kerne
 #pragma unroll
         for (int e = 0; e < 4; ++e) flush_in_place(k[e][u]);
       }
-      if (kt + nw < nt) load(kt + nw);  // in flight during this tile's chains
+      if (kPrefetch && kt + nw < nt) load(kt + nw);
       v16f acc, even, part;
       v16f d = products(q[0][0], k[0][0], neg0);
 #pragma unroll
