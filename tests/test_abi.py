@@ -10,6 +10,7 @@ import shutil
 import subprocess
 from pathlib import Path
 
+import numpy as np
 import pytest
 
 from opentars_amd import _lib
@@ -210,6 +211,30 @@ def test_codegen_has_no_fused_or_packed_fp32(tmp_path):
     assert not packed, sorted(set(packed))
     assert "scratch_" not in dis
     assert "v_mfma_i32_16x16x64_i8" in dis and "v_dot4" in dis
+
+
+def test_overlap_of_strided_rows_matches_a_walk_over_the_rows():
+    """The overlap refusal on strided matrices (equal strides, as columns of one buffer, and others)
+    against every pair of rows. tars_attention_noalloc checks overlaps before it refuses 65 rows of
+    4080 scores (E_RANGE), so no call here launches anything."""
+    import ctypes
+    lib = _lib.lib()
+    rng = np.random.default_rng(3)
+    M, nk, hd = 65, 4080, 64
+    one = lambda p: (ctypes.c_void_p * 1)(p)
+    seen = set()
+    for _ in range(3000):
+        ldq = 16 * int(rng.integers(16, 40))
+        ldatt = ldq if rng.random() < 0.6 else 16 * int(rng.integers(4, 80))
+        q = P + 16 * int(rng.integers(0, 6000))
+        att = P + 16 * int(rng.integers(0, 6000))
+        qr, ar = q + ldq * np.arange(M)[:, None], att + ldatt * np.arange(M)[None, :]
+        want = bool(((qr < ar + hd) & (ar < qr + 4 * hd)).any())
+        rc = lib.tars_attention_noalloc(one(q), ldq, one(P + 64 * MB), 4 * hd, one(P + 80 * MB), 4 * hd, 0, one(att), ldatt,
+                                        2, 0x3F800000, None, 0, None, 0, 1, M, nk, hd, 1, None)
+        assert rc == (_lib.E_OVERLAP if want else _lib.E_RANGE), (q - P, ldq, att - P, ldatt, want, rc)
+        seen.add((want, ldq == ldatt))
+    assert len(seen) == 4
 
 
 def test_fused_validation():
