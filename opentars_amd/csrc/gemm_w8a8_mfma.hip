@@ -6,7 +6,7 @@
 // and B use the same map: each dot product is then the exact sum over the instruction's 64 k.
 // Integer accumulation is exact, so K may be split across waves and summed in any order.
 //
-// Four kernel families:
+// Five kernel families:
 //  * mfma_chunk_kernel<KW, DB>: chunk rows (M <= 16) with one K block of whole 256-byte blocks: one
 //    16 x 16 output tile per workgroup, its weight and activation rows staged in LDS by each wave
 //    for its own share of K, the int32 partial tiles summed in LDS.
@@ -14,11 +14,13 @@
 //    that split its K range; every wave loads its share of all 16 (TM + TN) rows straight into
 //    MFMA operand registers, and the int32 partial tiles meet in LDS for the golden fp32 epilogue
 //    (or, for a K split, the per-block epilogue and the in-order fp32 adds across blocks). Used for
-//    K splits and for K blocks that are not a whole number of 256-byte stages.
+//    chunk rows and few prompt tiles of K blocks that are not a whole number of 256-byte stages.
 //  * mfma_tile_kernel<BM, BN, WM, WN, KS, S>: prompt rows. The tile's A and W rows are staged
 //    in LDS by direct global -> LDS loads of 4 rows x 256 bytes in a ring of S stages of KS bytes
 //    of K, every wave of the workgroup reading the shared operands from LDS; each wave owns whole
 //    16 x 16 output tiles over the full K, so there is no cross-wave reduction.
+//  * mfma_wide_kernel<BM, BN, WM, WN, S>: prompt rows, any K: larger tiles, stages of 128 bytes of K,
+//    one barrier per stage, operands double-buffered in registers.
 //  * mfma_panel_kernel<KQ>: prompt rows at K <= 1280 on 64 x 48 tiles. The whole K of the tile's
 //    rows is resident in LDS, loaded in three phases, and each 16-column block of the output is
 //    computed and stored as its weight rows land.
@@ -280,6 +282,25 @@ struct TileTail {
   float out_scale;
 };
 
+TileTail tile_tail(const MfmaArgs& a) {
+  TileTail tl{};
+  for (int i = 0; i < a.nseg; ++i) {
+    tl.W[i] = a.seg[i].W;
+    tl.K[i] = a.seg[i].K;
+    tl.koff[i] = a.seg[i].koff;
+  }
+  tl.nseg = a.nseg;
+  tl.bias = a.epi.bias;
+  tl.scol_per_tensor = a.epi.scol_per_tensor;
+  tl.act = a.epi.act;
+  tl.out = a.epi.out;
+  tl.out_scale = a.epi.out_scale;
+  return tl;
+}
+
+// QM_ROWCOL with fp32 output and neither bias nor activation (every K split)
+bool simple_epilogue(const RowColEpilogue& e) { return e.srow && !e.scol_per_tensor && !e.bias && e.act == 0 && e.out == 0; }
+
 // Stage st of this wave's L blocks into its ring slot (st % S).
 template <int L, int NW, int KS, int S>
 __device__ __forceinline__ void issue_stage(int8_t* lds, const int8_t* const (&src)[L], int wave, int st) {
@@ -469,6 +490,249 @@ hipError_t go_tile(const MfmaArgs& a, hipStream_t s) {
     else TARS_TILE(false, false);
   }
 #undef TARS_TILE
+  return hipGetLastError();
+}
+
+// ------------------------------------------------------------------------------------ wide tiles
+// Prompt rows on larger tiles and any K: stages of 128 bytes of K in a ring of S slots, operands
+// double-buffered in registers. Where the ring of mfma_tile_kernel is bound by latency (each stage waits
+// for its loads, then for its LDS reads, then multiplies), here a wave's 64-byte step reads the next
+// step's operands from LDS while its MFMAs run, and a stage takes one barrier:
+//   read step (st, 1); MFMAs of (st, 0); wait until stage st + 1 has landed, barrier (every wave's
+//   reads of stage st are done by then); issue stage st + S into slot st; read step (st + 1, 0); MFMAs of (st, 1).
+// The global -> LDS loads cover 8 rows x 128 bytes; row r of a 16-row group sits at byte 128 r, its
+// 16-byte chunk c in slot c ^ (r / 2): an MFMA operand read (one chunk of each of 16 rows) then touches
+// 16 distinct 16-byte bank groups (rows 2 i and 2 i + 1 take the two halves of the banks). A K that is no
+// multiple of 128 ends in a partial stage: its activation chunks past K read 16 zero bytes, its weight
+// chunks past K the row's last chunk (any bytes: they meet the zeros).
+//
+// Measured at M = 2048, K = N = 4096 on 128 x 256 tiles (one per CU): 8 waves of 64 x 64 outputs 41 us (1.68
+// POP/s; 95 us on the 64 x 64 ring tiles); 4 waves of 64 x 128 61 us (their accumulators and two operand
+// sets pass 256 registers and move through the others); the stages through registers and LDS writes
+// instead of direct loads 45 us; with neither loads nor LDS reads in the loop 33 us, where the matrix
+// cores' clock and the epilogue bound it. More ring slots than these changed nothing.
+__device__ const int4 kZeroChunk = {0, 0, 0, 0};
+
+template <int BM, int BN, int WM, int WN, int S, bool SIMPLE, bool KSPLIT>
+__global__ __launch_bounds__(64 * WM * WN, 2) void mfma_wide_kernel(const int8_t* A, const int8_t* W, const float* scol,
+                                                                 const float* srow, int lda, int K, int M, int N, int mt,
+                                                                 int ldy, void* Y, TileTail tl) {
+  constexpr int NW = WM * WN, NT = 64 * NW, TI = BM / 16 / WM, TJ = BN / 16 / WN, GA = BM / 16, G = (BM + BN) / 16;
+  constexpr int BLK = 2 * G, L = BLK / NW, SLOT = 1024 * BLK;
+  constexpr int TP = BN + 4;
+  // rows of the output tile staged through LDS at a time
+  constexpr int OM = BM * TP * 4 <= S * SLOT ? BM : BM / 2;
+  static_assert(BLK % NW == 0 && L * (S - 1) < 64 && S >= 3 && OM * TP * 4 <= S * SLOT && (OM == BM || WM % 2 == 0), "wide tile");
+  __shared__ __align__(16) int8_t lds[S * SLOT];
+  const v4i zero = {0, 0, 0, 0};
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int li = lane & 15, lg = lane >> 4;
+  // the tile order of mfma_tile_kernel: each XCD a contiguous range of tiles, M tiles fastest
+  const int G8 = mt * ((N + BN - 1) / BN);
+  const int b = blockIdx.x;
+  const int t = (G8 % 8 == 0) ? (b % 8) * (G8 / 8) + b / 8 : b;
+  const int m0 = (t % mt) * BM, n0 = (t / mt) * BN;
+
+  const int nseg = KSPLIT ? tl.nseg : 1;
+  v4i acc[TI][TJ];
+  // a K split adds its blocks' fp32 partials in block order, in registers
+  float chain[KSPLIT ? TI : 1][KSPLIT ? TJ : 1][4], sr[KSPLIT ? TI : 1], sc[KSPLIT ? TJ : 1][4];
+  if constexpr (KSPLIT) {
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) {  // a 16-column block past N reads the last one
+      const float4 c4 = *reinterpret_cast<const float4*>(scol + min(n0 + (wn * TJ + j) * 16, N - 16) + 4 * lg);
+      sc[j][0] = c4.x, sc[j][1] = c4.y, sc[j][2] = c4.z, sc[j][3] = c4.w;
+    }
+#pragma unroll
+    for (int i = 0; i < TI; ++i) sr[i] = *(srow ? srow + min(m0 + (wm * TI + i) * 16 + li, M - 1) : scol);
+    issue_fence();
+  }
+
+  for (int sgi = 0; sgi < nseg; ++sgi) {
+    const int8_t* Wg = (KSPLIT && sgi) ? tl.W[sgi] : W;
+    const int Kg = (KSPLIT && sgi) ? tl.K[sgi] : K;
+    const int ko = (KSPLIT && sgi) ? tl.koff[sgi] : 0;
+    const int NS = (Kg + 127) >> 7;
+    // Block i (rows 8 i .. + 7 of the tile, A's rows first) of each block this wave loads: a scalar base and the
+    // lane's 32-bit offset (row, 16-byte chunk). Rows past the matrix are clamped: they feed only outputs
+    // that are not stored.
+    const int8_t* const abase = A + static_cast<int64_t>(m0) * lda + ko;
+    const int8_t* const wbase = Wg + static_cast<int64_t>(n0) * Kg;
+    uint32_t off[L];
+    const int r8 = lane >> 3;
+#pragma unroll
+    for (int u = 0; u < L; ++u) {
+      const int i = wave + u * NW, g = i >> 1, r = 8 * (i & 1) + r8, c = 16 * ((lane & 7) ^ (r >> 1));
+      if (g < GA) off[u] = static_cast<uint32_t>(min(16 * g + r, M - 1 - m0)) * static_cast<uint32_t>(lda) + c;
+      else off[u] = static_cast<uint32_t>(min(16 * (g - GA) + r, N - 1 - n0)) * static_cast<uint32_t>(Kg) + c;
+    }
+    auto issue = [&](int st, int slot) __attribute__((always_inline)) {
+      const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_addr(lds) + SLOT * slot);
+      const int8_t *const ab = abase + 128 * st, *const wb = wbase + 128 * st;
+      if (128 * st + 128 <= Kg) {
+#pragma unroll
+        for (int u = 0; u < L; ++u) {
+          const int i = wave + u * NW;
+          ring_load16(i >> 1 < GA ? ab : wb, off[u], dst + 1024 * i);
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < L; ++u) {
+          const int i = wave + u * NW, r = 8 * (i & 1) + r8;
+          const int over = 128 * st + 16 * ((lane & 7) ^ (r >> 1)) - (Kg - 16);  // bytes past the row's last chunk
+          const int8_t* p = (i >> 1 < GA ? ab : wb) + off[u];
+          if (over > 0) p = i >> 1 < GA ? reinterpret_cast<const int8_t*>(&kZeroChunk) : p - over;
+          ring_load16(p, dst + 1024 * i);
+        }
+      }
+    };
+    auto read = [&](v4i (&fa)[TI], v4i (&fw)[TJ], int slot, int kb) __attribute__((always_inline)) {
+      const int8_t* s = lds + SLOT * slot + 128 * li + 16 * ((4 * kb + lg) ^ (li >> 1));
+#pragma unroll
+      for (int i = 0; i < TI; ++i) fa[i] = *reinterpret_cast<const v4i*>(s + 2048 * (wm * TI + i));
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) fw[j] = *reinterpret_cast<const v4i*>(s + 2048 * (GA + wn * TJ + j));
+    };
+    auto step = [&](const v4i (&fa)[TI], const v4i (&fw)[TJ]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) acc[i][j] = mfma(fw[j], fa[i], acc[i][j]);
+    };
+    if (KSPLIT && sgi) __builtin_amdgcn_s_barrier();  // every wave has read the last block's stages
+#pragma unroll
+    for (int st = 0; st < S; ++st)
+      if (st < NS) issue(st, st);
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) acc[i][j] = zero;
+    wait_stages_ahead<L, S - 1>(min(NS - 1, S - 1));
+    __builtin_amdgcn_s_barrier();
+    v4i fa0[TI], fw0[TJ], fa1[TI], fw1[TJ];
+    read(fa0, fw0, 0, 0);
+    int slot = 0;
+    for (int st = 0; st < NS; ++st) {
+      const int next = slot + 1 == S ? 0 : slot + 1;
+      read(fa1, fw1, slot, 1);
+      issue_fence();
+      step(fa0, fw0);
+      issue_fence();
+      if (st + 1 < NS) {
+        wait_lgkm0();
+        // stages st + 2 .. min(st + S - 1, NS - 1) may be outstanding
+        wait_stages_ahead<L, S - 2>(min(NS - 2 - st, S - 2));
+        __builtin_amdgcn_s_barrier();
+        if (st + S < NS) issue(st + S, slot);
+        read(fa0, fw0, next, 0);
+        issue_fence();
+      }
+      step(fa1, fw1);
+      issue_fence();
+      slot = next;
+    }
+    if constexpr (KSPLIT) {
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            float y = i2f(acc[i][j][v]);
+            if (srow) y = fmul(y, sr[i]);
+            y = fmul(y, sc[j][v]);
+            chain[i][j][v] = sgi == 0 ? y : fadd(chain[i][j][v], y);
+          }
+    }
+  }
+  // The sums (a K split: the outputs) go through LDS, OM rows of the tile at a time; there a thread owns
+  // four columns of every NT / (BN / 4)-th row, so it loads its column scales and biases once, and a row's
+  // consecutive 16-byte pieces are stored by consecutive threads.
+  int32_t* tile = reinterpret_cast<int32_t*>(lds);
+  constexpr int Q = BN / 4, RS = NT / Q;
+  static_assert(NT % Q == 0 && OM % RS == 0, "a thread keeps its columns");
+  const int cq = static_cast<int>(threadIdx.x) % Q, n = n0 + 4 * cq, nc = min(n, N - 4);
+  float4 c4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), b4 = c4;
+  if constexpr (!KSPLIT) {
+    if (SIMPLE || !tl.scol_per_tensor) c4 = *reinterpret_cast<const float4*>(scol + nc);
+    else c4 = make_float4(scol[0], scol[0], scol[0], scol[0]);
+    if (!SIMPLE && tl.bias) b4 = *reinterpret_cast<const float4*>(tl.bias + nc);
+  }
+#pragma unroll
+  for (int h = 0; h < BM / OM; ++h) {
+    __syncthreads();  // the stages (or the rows before) have been read
+    if (BM == OM || wm / (WM * OM / BM) == h) {
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) {
+          v4i o = acc[i][j];
+          if constexpr (KSPLIT) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) o[v] = static_cast<int>(fbits(chain[i][j][v]));
+          }
+          *reinterpret_cast<v4i*>(tile + ((wm * TI + i) * 16 - h * OM + li) * TP + (wn * TJ + j) * 16 + 4 * lg) = o;
+        }
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int r = static_cast<int>(threadIdx.x) / Q; r < OM; r += RS) {
+      const int m = m0 + h * OM + r;
+      const v4i o = *reinterpret_cast<const v4i*>(tile + r * TP + 4 * cq);
+      const float srm = KSPLIT ? 0.0f : *(srow ? srow + min(m, M - 1) : scol);
+      float y[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float sv = v == 0 ? c4.x : v == 1 ? c4.y : v == 2 ? c4.z : c4.w;
+        const float bv = v == 0 ? b4.x : v == 1 ? b4.y : v == 2 ? b4.z : b4.w;
+        const int ov = o[v];
+        if constexpr (KSPLIT) {
+          y[v] = ffrom(static_cast<uint32_t>(ov));
+        } else if constexpr (SIMPLE) {
+          y[v] = fmul(fmul(i2f(ov), srm), sv);
+        } else {
+          y[v] = i2f(ov);
+          if (srow) y[v] = fmul(y[v], srm);
+          y[v] = fmul(y[v], sv);
+          if (tl.bias) y[v] = fadd(y[v], bv);
+          y[v] = act_fn(y[v], tl.act);
+        }
+      }
+      if (m < M && n < N) {
+        if constexpr (SIMPLE || KSPLIT) {
+          *reinterpret_cast<float4*>(static_cast<char*>(Y) + static_cast<int64_t>(m) * ldy + 4 * n) =
+              make_float4(ftz(y[0]), ftz(y[1]), ftz(y[2]), ftz(y[3]));
+        } else {
+          store_out4(Y, static_cast<int64_t>(m) * ldy, n, tl.out, y, tl.out_scale);
+        }
+      }
+    }
+  }
+}
+
+template <int BM, int BN, int WM, int WN, int S>
+hipError_t go_wide(const MfmaArgs& a, hipStream_t s) {
+  static_assert(static_cast<size_t>(S) * (BM + BN) * 128 <= 163840, "stage ring exceeds 160 KiB of LDS");
+  const int mt = (a.M + BM - 1) / BM, nt = (a.N + BN - 1) / BN;
+  const TileTail tl = tile_tail(a);
+  const bool simple = simple_epilogue(a.epi);
+  const int8_t* A = a.A + a.seg[0].koff;
+  const int lda = static_cast<int>(a.lda), ldy = static_cast<int>(a.ldy);
+  const dim3 grid(mt * nt), block(64 * WM * WN);
+#define TARS_WIDE(SIMPLE, KSPLIT)                                                                                  \
+  hipLaunchKernelGGL((mfma_wide_kernel<BM, BN, WM, WN, S, SIMPLE, KSPLIT>), grid, block, 0, s, A, a.seg[0].W,      \
+                     a.epi.scol, a.epi.srow, lda, a.seg[0].K, a.M, a.N, mt, ldy, a.Y, tl)
+  if (a.nseg > 1) {
+    // the larger tiles have no registers left for the chain of a K split's partials
+    if constexpr (BM * BN <= 64 * 128) TARS_WIDE(true, true);
+    else return hipErrorInvalidValue;
+  } else {
+    if (simple) TARS_WIDE(true, false);
+    else TARS_WIDE(false, false);
+  }
+#undef TARS_WIDE
   return hipGetLastError();
 }
 
@@ -775,23 +1039,27 @@ hipError_t go_chunk(const MfmaArgs& a, hipStream_t s) {
 // -> 2.92 / 3.62 us, M = 16 4.48 / 6.61 -> 3.10 / 4.16 us against the direct kernel (its 16-row x
 // 64-byte register loads touch twice the cache lines per instruction); the direct kernel with 8
 // waves over K otherwise.
-// Prompt rows, when every K block is a whole number of stages (K a multiple of 256): the LDS tile
-// kernel, its tile chosen by measurement on MI355X with the weights cold, bit-identical across
-// tiles; the direct kernel's 32 x 32 tiles with 4 waves over K otherwise.
-//  * 64 x 48 tiles (4 waves of 16 x 48, 256-byte stages, 3 slots) when they give one to 1.25
-//    workgroups per CU: M=256 K=1024 N=3072 7.5 -> 5.5 us (the 64 x 64 / 16-row-load tiles before;
-//    4 / 5 slots 5.70 / 5.89 us against 5.40, 512-byte stages in 2 slots 5.41 us); with one K block
-//    of at most 1280 the panel form of the same tiles instead: K = 1024 5.41 -> 4.71 us (5.04 us
-//    with block 1's store issued before the last wait and the epilogue operands before the first
-//    loads; block 2 in two K halves 4.86 us), K = 256 / 512 / 768 / 1280 at N = 3072: 3.91 / 4.45 /
-//    4.92 / 5.89 -> 3.63 / 3.96 / 4.27 / 5.26 us;
-//  * 64 x 64 tiles (4 waves of 32 x 32, 256-byte stages, 3 slots) when they give 512 or more:
-//    M=1024 K=1024 N=3072 16.5 -> 15.8 us;
-//  * 32 x 32 tiles (4 waves of 16 x 16) with 512-byte stages in 3 slots when K is a multiple of
-//    1024 and they give at most 1.25 workgroups per CU: M=256 K=3072 N=1024 8.6 -> 5.9 us with
-//    1024-byte stages in 2 slots, 5.76 us with these (K = 1024 / 2048 / 4096 at N = 1024: 4.04 /
-//    4.86 / 6.72 -> 3.77 / 4.77 / 6.68 us; 512-byte stages in 4 slots 0.1 - 0.3 us slower);
-//  * 32 x 32 tiles with 256-byte stages in 3 slots otherwise: M=64 K=1024 N=3072 5.2 -> 3.8 us.
+// Prompt rows (M > 16): the tile by how many of them the problem gives (256 CUs), every line where the two
+// sides were measured equal over M = 24 - 3000 and ten (K, N) pairs from 1024 x 3072 to 4096 x 4096, weights
+// cold; the results are the same bits for every tile.
+//  * 128 x 256 wide tiles (8 waves) from 192 of them when the last round of 256 is at least 4/5 full (3/4
+//    from K = 2048, where a tile's fill matters less): M = 2048, K = 4096, N = 4096 95 -> 41 us (64 x 64 ring
+//    tiles before; 64 x 128 wide 51 us), M = 3000, K = 1024, N = 3072 (288 tiles: 56%) 33 us against 27 on the next;
+//  * with K blocks of whole 256-byte stages: the 64 x 48 tiles at 192 to 256 of them (in the panel form with one
+//    K block of at most 1280): M = 256, K = 1024, N = 3072 5.0 us (64 x 64 wide 5.7; a second round for a few
+//    tiles is what they lose by: M = 260 7.5 against 5.6); the 32 x 32 ring with 512-byte stages at most 256 of
+//    them and K a multiple of 1024 (M = 256, K = 3072, N = 1024 6.2 us, 32 x 64 wide 8.4);
+//  * 64 x 128 wide tiles from 192 of them: M = 1024, K = 1024, N = 3072 14.9 -> 10.7 us, M = 777, K = 4096, N = 4096
+//    43 -> 24 us, M = 512, K = 1152, N = 6912 35.6 -> 12.0 us (32 x 32 direct tiles before). With GELU and the
+//    activations after it the epilogue weighs as much as the sums, and below 512 tiles a CU with two of them
+//    holds the others up: M = 333, K = 1152, N = 6912 28 us, 22 us on 64 x 64 wide tiles;
+//  * whole 256-byte stages and at most 512 32 x 32 tiles: the 32 x 32 ring with 256-byte stages (M = 512,
+//    K = 3072, N = 1024 8.2 us, 32 x 64 wide 8.6; at 640 tiles, M = 130, K = N = 4096, 19.6 against 12.0);
+//  * 64 x 64 wide tiles from 192 of them (M = 777, K = 3072, N = 1024 16.9 -> 10.4 us), else 32 x 64 wide tiles
+//    (M = 64, K = 1152, N = 6912 9.0 -> 5.3 us);
+//  * the direct kernel's 32 x 32 tiles with 4 waves over K for few tiles of a long K that is not whole
+//    stages (M = 20, K = 2064, N = 2048 6.2 us, 32 x 64 wide 6.8) and for row strides the LDS kernels' 32-bit
+//    offsets do not cover. A K split runs the same rules without the 128 x 256 tiles.
 bool whole_stages(const MfmaArgs& a, int ks) {
   for (int i = 0; i < a.nseg; ++i)
     if (a.seg[i].K % ks) return false;
@@ -811,10 +1079,15 @@ hipError_t run(const MfmaArgs& a, hipStream_t s) {
     }
     return go_direct<1, 1, 8, 1>(a, s);
   }
-  // the LDS tile kernels take 32-bit row strides; the direct kernel any
-  if (!whole_stages(a, 256) || a.lda > INT32_MAX || a.ldy > INT32_MAX) return go_direct<2, 2, 4, 1>(a, s);
-  const int64_t t48 = tiles(a, 64, 48), t32 = tiles(a, 32, 32);
-  if (t48 >= 192 && t48 <= 320) {
+  // the LDS kernels take 32-bit offsets inside a tile's rows; the direct kernel any strides
+  if (a.lda >= (1 << 24) || a.ldy > INT32_MAX) return go_direct<2, 2, 4, 1>(a, s);
+  const bool whole = whole_stages(a, 256);
+  const int64_t tw = tiles(a, 128, 256), tc = tiles(a, 64, 128), t48 = tiles(a, 64, 48), t64 = tiles(a, 64, 64),
+                t32 = tiles(a, 32, 32);
+  const int64_t rounds = (tw + 255) / 256 * 256;  // 128 x 256 tiles that whole rounds would hold
+  if (a.nseg == 1 && tw >= 192 && (5 * tw >= 4 * rounds || (a.seg[0].K >= 2048 && 4 * tw >= 3 * rounds)))
+    return go_wide<128, 256, 2, 4, 3>(a, s);
+  if (whole && t48 >= 192 && t48 <= 256) {
     if (a.nseg == 1 && a.seg[0].K <= 1280) {
       switch (a.seg[0].K / 256) {
         case 1: return go_panel<1>(a, s);
@@ -826,9 +1099,14 @@ hipError_t run(const MfmaArgs& a, hipStream_t s) {
     }
     return go_tile<64, 48, 4, 1, 256, 3>(a, s);
   }
-  if (tiles(a, 64, 64) >= 512) return go_tile<64, 64, 2, 2, 256, 3>(a, s);
-  if (t32 <= 320 && whole_stages(a, 1024)) return go_tile<32, 32, 2, 2, 512, 3>(a, s);
-  return go_tile<32, 32, 2, 2, 256, 3>(a, s);
+  if (t32 <= 256 && whole_stages(a, 1024)) return go_tile<32, 32, 2, 2, 512, 3>(a, s);
+  if (tc >= 192 && (tc >= 512 || a.epi.act < 3)) return go_wide<64, 128, 2, 4, 3>(a, s);
+  if (whole && t32 <= 512) return go_tile<32, 32, 2, 2, 256, 3>(a, s);
+  if (t64 >= 192) return go_wide<64, 64, 2, 4, 4>(a, s);
+  int longest = 0;
+  for (int i = 0; i < a.nseg; ++i) longest = a.seg[i].K > longest ? a.seg[i].K : longest;
+  if (tiles(a, 32, 64) < 96 && longest > 1280) return go_direct<2, 2, 4, 1>(a, s);
+  return go_wide<32, 64, 2, 2, 4>(a, s);
 }
 
 }  // namespace

@@ -35,11 +35,32 @@ __device__ __forceinline__ void stage16(const void* src, void* dst) {
   __builtin_amdgcn_global_load_lds(src, TARS_LDS(dst), 16, 0, 0);
 }
 
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>(TARS_LDS(p)));
+}
+
+// One direct global -> LDS load (global_load_lds_dwordx4; dst is the wave-uniform LDS
+// address of the 1 KiB block), written as assembly that sets M0 itself. The compiler does not see
+// it as a write to LDS, so it adds no wait for every such load in flight before a later LDS read
+// (which it does for the builtin, not knowing which bytes it writes); the kernel's own waits and
+// barriers order the ring instead. No other code in the kernel keeps a value in M0.
+__device__ __forceinline__ void ring_load16(const void* src, uint32_t dst) {
+  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(dst) : "memory");
+}
+
+// The same from a scalar base and a 32-bit lane offset.
+__device__ __forceinline__ void ring_load16(const void* base, uint32_t off, uint32_t dst) {
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(dst) : "memory");
+}
+
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit count");
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
+
+// Waits until every LDS access of this wave is done (lgkmcnt(0)).
+__device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xC07F); }
 
 // Waits until at most L * ahead of this wave's vector loads are outstanding: a ring of stages of L
 // loads each, `ahead` (uniform, 0..A) of them issued after the one about to be read.

@@ -594,19 +594,6 @@ __global__ __launch_bounds__(256) void fdot_nn_kernel(FdotArgs a) {
 // ops leave them.
 constexpr int kAttnSlots = 6, kAttnStageBytes = 8192;
 
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>(TARS_LDS(p)));
-}
-
-// One direct global -> LDS load of the V ring (global_load_lds_dwordx4; dst is the wave-uniform LDS
-// address of the 1 KiB block), written as assembly that sets M0 itself. The compiler does not see
-// it as a write to LDS, so it adds no wait for every such load in flight before a later LDS read
-// (which it does for the builtin, not knowing which bytes it writes); the ring's stage waits and
-// barriers order the ring instead. No other code in the kernel keeps a value in M0.
-__device__ __forceinline__ void ring_load16(const void* src, uint32_t dst) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(dst) : "memory");
-}
-
 // The score chains of Q query rows qv against KF keys whose K elements (this lane's U of each row)
 // are in kv, unflushed (qv is flushed) and checked; recomputed with the contract's flushes when a
 // key element or a partial sum lies in (0, 2^-100) in magnitude (a subnormal product is then

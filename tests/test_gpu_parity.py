@@ -607,6 +607,47 @@ def test_w8a8_random_panels(seed):
     assert same(host(y), want), ((M, N, qm, act, out), mismatch(host(y), want))
 
 
+# one ragged case per wide tile and kind of K: whole 128-byte stages, a partial last stage, K shorter than a
+# stage, and one, two and more stages than the ring holds (128 x 256, 64 x 128, 64 x 64 and 32 x 64 tiles in
+# that order; the 64 x 64 tiles by GELU where the others take none)
+@pytest.mark.parametrize("M,N,K,act,out,qm", [
+    (300, 17664, 144, ACT_NONE, OUT_FP32, "rowcol"), (257, 18688, 256, ACT_SILU, OUT_BF16, "channel"),
+    (385, 13232, 528, ACT_NONE, OUT_INT8, "rowcol"),
+    (65, 12304, 16, ACT_NONE, OUT_FP32, "rowcol"), (128, 12288, 384, ACT_RELU, OUT_INT8, "tensor"),
+    (100, 12400, 656, ACT_NONE, OUT_FP32, "rowcol"),
+    (129, 4112, 48, ACT_GELU, OUT_FP32, "rowcol"), (192, 4096, 640, ACT_SOFTPLUS, OUT_INT8, "rowcol"),
+    (200, 4112, 1168, ACT_GELU, OUT_BF16, "channel"),
+    (17, 80, 112, ACT_NONE, OUT_FP32, "rowcol"), (33, 1040, 128, ACT_SILU, OUT_BF16, "tensor"),
+    (97, 2064, 1152, ACT_NONE, OUT_FP32, "rowcol"),
+])
+def test_wide_tiles(M, N, K, act, out, qm):
+    rng = np.random.default_rng(M * 7 + K)
+    A = np.ascontiguousarray(rng.integers(-128, 128, (M, K + 48), dtype=np.int8))
+    W = rng.integers(-128, 128, (N, K), dtype=np.int8)
+    sc = rng.uniform(1e-4, 3e-2, N).astype(f32)
+    sc = sc[:1] if qm == "tensor" else sc
+    srow = rng.uniform(0.1, 2.0, M).astype(f32) if qm == "rowcol" else None
+    b = rng.normal(0, 2, N).astype(f32)
+    osc = f32(5.0) if out == OUT_INT8 else None
+    pitch = K + 48                                    # strided activation rows; the bytes past K differ
+    y = ops.gemm_rowcol(cuda(A).view(M, pitch)[:, :K], None if srow is None else cuda(srow), cuda(W), cuda(sc), cuda(b),
+                        act=act, out=out, out_scale=osc)
+    want = G.gemm_rowcol(np.ascontiguousarray(A[:, :K]), srow, W, sc, b, act=act, out=out, out_scale=osc)
+    assert same(host(y), want), mismatch(host(y), want)
+
+
+@pytest.mark.parametrize("M,N,blocks", [(100, 12304, [128, 144, 16]), (200, 6160, [512, 256]), (130, 4112, [48, 1040]),
+                                        (40, 1040, [272, 128])])
+def test_ksplit_wide_tiles(M, N, blocks):
+    _, q, s, _, _, _ = w8_inputs(M, M, 16, sum(blocks))
+    rng = np.random.default_rng(N)
+    Ws = [rng.integers(-127, 128, (N, k), dtype=np.int8) for k in blocks]
+    sc = rng.uniform(1e-3, 1e-2, N).astype(f32)
+    y = ops.gemm_rowcol_ksplit(cuda(q), cuda(s), [cuda(w) for w in Ws], cuda(sc))
+    want = G.gemm_rowcol_ksplit(q, s, Ws, sc)
+    assert same(host(y), want), mismatch(host(y), want)
+
+
 @pytest.mark.parametrize("seed", range(24))
 def test_ksplit_random_blocks(seed):
     """The K split over random block counts (1 to 5) and block widths (multiples of 16, total K
