@@ -1026,86 +1026,101 @@ __global__ __launch_bounds__(256) void attn_split_scores_kernel(AttnArgs a) {
 
 // The causal softmax (ROW_SOFTMAX) of Q rows of scores in LDS, in place and side by side: row i at
 // sp + i * ldp is query row i % M of its head, with min(nk, causal_k + i % M) valid keys (nk when
-// causal_k is 0). Every step of every row is spread over the whole workgroup, each thread taking
-// the same element of every row together (independent work for the latency of exp_f), and the
-// rows' 16-lane sums run together (lds_sum16_rows); each row's values are softmax_lds's. Rows from
-// pr_first on also go to pr (row i - pr_first at ldpr bytes) when pr is not null. Returns whether
-// one of this thread's probabilities is above 1 or NaN.
-template <int Q>
-__device__ __forceinline__ int softmax_rows_lds(float* sp, int ldp, int M, int nk, int causal_k, int pr_first,
-                                                float* pr, int64_t ldpr, uint32_t (*red)[4], float* bcast) {
-  const int t = threadIdx.x, lane = t & 63;
-  int V[Q];
-#pragma unroll
-  for (int i = 0; i < Q; ++i) V[i] = causal_k > 0 ? min(nk, causal_k + i % M) : nk;
+// causal_k is 0). Each row has NT / 64 / Q waves of the workgroup (every thread taking its element of
+// all rows cost 4 rows of 104 keys 0.4 us: exp_f is some sixty instructions, and most lanes had none);
+// the rows' 16-lane sums run together (lds_sum16_rows); each row's values are softmax_lds's. Rows from
+// pr_first on also go to pr (row i - pr_first at ldpr bytes) when pr is not null.
+template <int Q, int NT>
+__device__ __forceinline__ void softmax_rows_lds(float* sp, int ldp, int M, int nk, int causal_k, int pr_first,
+                                                float* pr, int64_t ldpr, uint32_t (&red)[NT / 64], float* bcast) {
+  constexpr int W = NT / 64 / Q, T = 64 * W;  // waves and threads per row
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int i = wave / W, t = static_cast<int>(threadIdx.x) - i * T;
+  const bool mine = i < Q;  // (a last wave can be left over)
+  const int V = causal_k > 0 ? min(nk, causal_k + i % M) : nk;
+  float* const s = sp + i * ldp;
   __syncthreads();  // the rows are complete
-  // the maximum key of each row's valid keys, a NaN counting as 0xFFFFFFFF (above every other key:
-  // +inf's is 0xFF800000), branch-free, then one whole-wave maximum per row
-  uint32_t key[Q];
-#pragma unroll
-  for (int i = 0; i < Q; ++i) key[i] = 0;
-  for (int j = t; j < nk; j += 256) {
-#pragma unroll
-    for (int i = 0; i < Q; ++i) {
-      const float x = sp[i * ldp + j];
-      const uint32_t k = is_nan(x) ? 0xFFFFFFFFu : fmax_key(x);
-      key[i] = j < V[i] ? max(key[i], k) : key[i];
+  // the maximum key of the row's valid keys, a NaN counting as 0xFFFFFFFF (above every other key:
+  // +inf's is 0xFF800000), branch-free, then one whole-wave maximum
+  if (mine) {
+    uint32_t key = 0;
+    for (int j = t; j < V; j += T) {
+      const float x = s[j];
+      key = max(key, is_nan(x) ? 0xFFFFFFFFu : fmax_key(x));
     }
-  }
-#pragma unroll
-  for (int i = 0; i < Q; ++i) {
-    key[i] = wave_max_u32(key[i]);
-    if (lane == 0) red[i][t >> 6] = key[i];
+    key = wave_max_u32(key);
+    if (lane == 0) red[wave] = key;
   }
   __syncthreads();
-  float nmx[Q];
+  if (mine) {
+    uint32_t k = red[i * W];
 #pragma unroll
-  for (int i = 0; i < Q; ++i) {
-    const uint32_t k4 = max(max(red[i][0], red[i][1]), max(red[i][2], red[i][3]));
-    nmx[i] = fneg(k4 == 0xFFFFFFFFu ? ffrom(kCanonNaN) : fmax_from_key(k4));
-  }
-  for (int j = t; j < nk; j += 256) {
-    float e[Q];
-#pragma unroll
-    for (int i = 0; i < Q; ++i) e[i] = exp_f(fadd(sp[i * ldp + j], nmx[i]));
-#pragma unroll
-    for (int i = 0; i < Q; ++i) sp[i * ldp + j] = j < V[i] ? e[i] : 0.0f;
+    for (int w = 1; w < W; ++w) k = max(k, red[i * W + w]);
+    const float nmx = fneg(k == 0xFFFFFFFFu ? ffrom(kCanonNaN) : fmax_from_key(k));
+#pragma unroll 2
+    for (int j = t; j < nk; j += T) {
+      const float e = exp_f(fadd(s[j], nmx));
+      s[j] = j < V ? e : 0.0f;
+    }
   }
   lds_sum16_rows<false, true>(sp, ldp, Q, nk, bcast);  // exp_f values: 0, normal, inf or NaN
-  float r[Q];
-#pragma unroll
-  for (int i = 0; i < Q; ++i) r[i] = recip_f(bcast[i]);
-  int above1 = 0;
-  for (int j = t; j < nk; j += 256) {
-#pragma unroll
-    for (int i = 0; i < Q; ++i) {
-      const float p = fmul(sp[i * ldp + j], r[i]);
-      sp[i * ldp + j] = p;
-      above1 |= !(p <= 1.0f);
+  if (mine) {
+    const float r = recip_f(bcast[i]);
+#pragma unroll 2
+    for (int j = t; j < nk; j += T) {
+      const float p = fmul(s[j], r);
+      s[j] = p;
       if (pr && i >= pr_first) store_out(pr, (i - pr_first) * ldpr, j, 0, p, 0.0f);
     }
   }
-  return above1;
 }
 
 // Split form, second kernel: workgroup (hg, c) loads the scratch scores of the Q = group * M query
-// rows of head group hg (Q consecutive scratch rows) into LDS by direct loads, then issues the
-// first stages of a ring of direct loads of V's columns [32 c, 32 c + 32), runs the Q softmaxes
-// side by side (the same probabilities in every workgroup of the group; workgroup 0 of the last
-// head's group stores that head's), then the P V chains of those columns for every query row,
-// one thread per (query row, column).
-template <int HD, bool VHALF, int Q>
-__global__ __launch_bounds__(256) void attn_split_pv_kernel(AttnArgs a) {
-  constexpr int DS = kAttnSplitCols, ES = VHALF ? 2 : 4;
-  constexpr int ROWB = DS * ES;                      // bytes of a V row's columns (128 / 64)
-  constexpr int LPR = ROWB / 16;                     // lanes per row in a 1 KiB load
-  constexpr int SB = 8192, SR = SB / ROWB;           // rows per stage
-  constexpr int SLOTS = 5, L = SB / 1024 / 4;        // 1 KiB loads per wave per stage (2)
-  static_assert(HD % DS == 0 && 1024 % ROWB == 0 && kAttnSplitProbs % 256 == 0, "split attention shape");
-  __shared__ __align__(16) float sp[kAttnSplitProbs];
-  __shared__ __align__(16) int8_t ring[SLOTS * SB];
-  __shared__ uint32_t red[kAttnSplitMaxQ][4];
-  __shared__ float bcast[kAttnSplitMaxQ];
+// rows of head group hg (Q consecutive scratch rows) into LDS, runs the Q softmaxes side by side (the
+// same probabilities in every workgroup of the group; workgroup 0 of the last head's group stores that
+// head's), then the P V chains of columns [32 c, 32 c + 32) for every query row, one lane per (query
+// row, column).
+//
+// A chain is one dependent add per key, in key order, and a wave issues a vector instruction every 4.9
+// cycles at best, so whatever else the chain's wave does per key adds to the kernel's time. Here it does
+// nothing but add: eight producer waves form the products of a stage of 64 keys (a lane takes one column
+// of four keys for all Q rows), into one of two LDS buffers laid out so that a chain's lane reads four
+// keys with one 16-byte load, 32 keys ahead of its adds and across the stages' barriers; V comes to the
+// producers' registers AHEAD stages early, the first ones before the softmax. Products are formed
+// with subnormals kept and added with them flushed, which is the contract's fadd(acc, fmul(p, v)) in one
+// instruction each without a check (see attn_rows.hip); a key past the last one gives a product of -0,
+// which leaves every sum as it is.
+// Measured on MI355X, 16 heads of 128 over 8 K / V heads: 2048 keys 201 us with the chains' wave also
+// multiplying and checking each sum for the flushes (its inputs redo stages whose sums are tiny) -> 18 us
+// (27 us before the V loads' waits counted exactly); a whole attention call there 207 -> 21.5 us, a decode
+// step at 250 keys 1.2 us less per layer.
+constexpr int kPvStage = 64, kPvProducers = kPvStage / 4 * kAttnSplitCols;
+constexpr int pv_chain_waves(int Q) { return (Q * kAttnSplitCols + 63) / 64; }
+constexpr int pv_threads(int Q) { return kPvProducers + 64 * pv_chain_waves(Q); }
+
+// fp32 subnormals kept / flushed (MODE bits 4-5) from here on; values that cross a switch pass through
+// tie(), which the compiler keeps in order with it.
+__device__ __forceinline__ void keep_denorms() { __builtin_amdgcn_s_setreg(1 | (4 << 6) | (1 << 11), 3); }
+__device__ __forceinline__ void flush_denorms() { __builtin_amdgcn_s_setreg(1 | (4 << 6) | (1 << 11), 0); }
+__device__ __forceinline__ void tie(float& x) { asm volatile("" : "+v"(x)); }
+
+// A workgroup barrier that orders LDS only: V loads stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <bool VHALF, int Q, int AHEAD>
+__global__ __launch_bounds__(pv_threads(Q)) void attn_split_pv_kernel(AttnArgs a) {
+  constexpr int DS = kAttnSplitCols, ES = VHALF ? 2 : 4, SK = kPvStage, NT = pv_threads(Q);
+  constexpr int LD = SK + 4;  // 4 * odd: the 16-byte reads and writes of consecutive chains spread over the banks
+  constexpr int kBlock = SK / 2;
+  static_assert(kPvProducers == SK / 4 * DS, "one producer thread per column and four keys");
+  __shared__ __align__(16) float sp[kAttnSplitProbs + SK];
+  __shared__ __align__(16) float prod[2][Q * DS * LD];
+  __shared__ uint32_t red[NT / 64];
+  __shared__ float bcast[Q];
   const int hg = blockIdx.x, c = blockIdx.y, t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int G = a.group, M = a.M, nk = a.nk;  // G * M == Q
@@ -1115,58 +1130,129 @@ __global__ __launch_bounds__(256) void attn_split_pv_kernel(AttnArgs a) {
   __asm__ volatile("" : : "s"(a.v[hg * G]), "s"(a.ldv), "s"(a.scratch), "s"(a.ld_scratch), "s"(a.causal_k),
                    "s"(a.pr), "s"(a.ldpr), "s"(a.att[hg * G]), "s"(a.ldatt), "s"(a.out), "s"(a.out_scale));
   const int ldp = static_cast<int>(a.ld_scratch);
-  const int NS = (nk + SR - 1) / SR;
-  const char* vbase = static_cast<const char*>(a.v[hg * G]) + c * ROWB;
-  auto issue = [&](int st) {
-    int8_t* slot = ring + SB * (st % SLOTS);
+  const int NS = (nk + SK - 1) / SK;
+  const bool producer = wave < kPvProducers / 64;
+  // the Q score rows (Q ldp floats, contiguous in the scratch): at most two 16-byte loads per thread
+  const float4* srows = reinterpret_cast<const float4*>(a.scratch + static_cast<int64_t>(hg) * Q * a.ld_scratch);
+  constexpr int SL = (kAttnSplitProbs / 4 + NT - 1) / NT;
+  const int n4 = Q * ldp / 4;
+  float4 sv[SL];
 #pragma unroll
-    for (int u = 0; u < L; ++u) {
-      const int i = wave + 4 * u;
-      const int row = min(st * SR + i * (1024 / ROWB) + lane / LPR, nk - 1);
-      ring_load16(vbase + static_cast<int64_t>(row) * a.ldv + 16 * (lane % LPR),
-                  __builtin_amdgcn_readfirstlane(lds_addr(slot + i * 1024)));
+  for (int i = 0; i < SL; ++i) sv[i] = srows[min(t + NT * i, n4 - 1)];
+  // this producer's four keys of a stage: rows 4 quad .. 4 quad + 3, column d
+  const int quad = t / DS, d = t % DS;
+  using Elem = std::conditional_t<VHALF, uint16_t, uint32_t>;
+  using GlobalBytes = const __attribute__((address_space(1))) char;  // (a generic load would count as an LDS access too)
+  using GlobalElem = const __attribute__((address_space(1))) Elem;
+  Elem vq[AHEAD][4];
+  GlobalBytes* vb = (GlobalBytes*)a.v[hg * G];
+  const int64_t vcol = (c * DS + d) * ES;
+  int64_t off[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) off[k] = (4 * quad + k) * a.ldv + vcol;
+  // (no load is conditional, so that the waits before a stage's use count exactly: keys past the end load
+  // the last row again, stages past the end the first)
+  auto load = [&](Elem (&v)[4], int st) __attribute__((always_inline)) {
+    GlobalBytes* p[4];
+    if ((st + 1) * SK <= nk) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) p[k] = vb + st * SK * a.ldv + off[k];
+    } else if (st >= NS) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) p[k] = vb + vcol;
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) p[k] = vb + min(st * SK + 4 * quad + k, nk - 1) * a.ldv + vcol;
     }
-  };
-  // the Q score rows (4 Q ldp bytes, contiguous in the scratch) in 1 KiB blocks; a block's lanes
-  // past the end read the last 16 bytes again (into LDS past the rows, inside sp)
-  const int sbytes = 4 * Q * ldp;
-  const char* sbase = reinterpret_cast<const char*>(a.scratch + static_cast<int64_t>(hg) * Q * a.ld_scratch);
-  for (int b = wave; 1024 * b < sbytes; b += 4)
-    ring_load16(sbase + min(1024 * b + 16 * lane, sbytes - 16), __builtin_amdgcn_readfirstlane(lds_addr(sp + 256 * b)));
 #pragma unroll
-  for (int st = 0; st < SLOTS - 1; ++st)
-    if (st < NS) issue(st);
-  wait_stages_ahead<L, SLOTS - 1>(min(NS, SLOTS - 1));  // this wave's score blocks have landed
+    for (int k = 0; k < 4; ++k) v[k] = *(GlobalElem*)p[k];
+  };
+  auto put_scores = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < SL; ++i) reinterpret_cast<float4*>(sp)[min(t + NT * i, n4 - 1)] = sv[i];
+  };
+  if (producer) {
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) load(vq[i], i);
+    put_scores();
+  } else {
+    put_scores();
+  }
   const int pr_first = hg == gridDim.x - 1 && c == 0 ? (G - 1) * M : Q;
-  const int above1 = softmax_rows_lds<Q>(sp, ldp, M, nk, a.causal_k, pr_first, a.pr, a.ldpr, red, bcast);
-  wait_vmcnt<0>();  // the first V stages have landed; nothing else outstanding before the ring's counts
-  // V elements need their own test only when fp32 and some probability is above 1 or NaN (as in
-  // attn_kernel)
-  const bool vtest = __syncthreads_or(above1) && !VHALF;
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");  // the slots' reads stay after the barrier
-  const int i = t / DS, d = t % DS;
-  const bool active = i < Q;
-  float acc = 0.0f;
-  if (NS <= SLOTS - 1) {
-    // every stage was issued before the softmax, has landed (each wave's wait_vmcnt<0> above) and is
-    // visible (the barrier): the stages sit in consecutive slots, so the chains run over all keys in
-    // one pipelined pass, without the per-stage waits and barrier pairs
-    if (active) acc = pv_stage<VHALF, SR, ROWB>(acc, ring, d, sp + i * ldp, nk, vtest);
-    if (active) store_out(a.att[hg * G + i / M], (i % M) * a.ldatt, c * DS + d, a.out, chain_end(acc), a.out_scale);
+  softmax_rows_lds<Q, NT>(sp, ldp, M, nk, a.causal_k, pr_first, a.pr, a.ldpr, red, bcast);
+  lds_barrier();
+  if (producer) {
+    const int ldp4 = ldp >> 2;
+    auto stage = [&](Elem (&e)[4], int st, auto tail) __attribute__((always_inline)) {
+      float v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if constexpr (VHALF) v[k] = fp16_to_f32_keep_nan(e[k]);
+        else v[k] = ftz(ffrom(e[k]));
+      }
+      if constexpr (!decltype(tail)::value) load(e, st + AHEAD);
+      const int j = st * SK + 4 * quad;
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const float4 p = reinterpret_cast<const float4*>(sp)[q * ldp4 + (j >> 2)];
+        float4 x = make_float4(__fmul_rn(p.x, v[0]), __fmul_rn(p.y, v[1]), __fmul_rn(p.z, v[2]), __fmul_rn(p.w, v[3]));
+        if constexpr (decltype(tail)::value) {
+          x.x = j < nk ? x.x : -0.0f;
+          x.y = j + 1 < nk ? x.y : -0.0f;
+          x.z = j + 2 < nk ? x.z : -0.0f;
+          x.w = j + 3 < nk ? x.w : -0.0f;
+        }
+        *reinterpret_cast<float4*>(&prod[st & 1][(q * DS + d) * LD + 4 * quad]) = x;
+      }
+      lds_barrier();  // stage st is complete, stage st - 1 has been read
+    };
+    int s0 = 0;
+    for (; s0 + AHEAD < NS; s0 += AHEAD)
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) stage(vq[i], s0 + i, std::false_type{});
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i)
+      if (s0 + i < NS) stage(vq[i], s0 + i, std::true_type{});
     return;
   }
+  __builtin_amdgcn_s_setprio(3);
+  const int chain = (wave - kPvProducers / 64) * 64 + lane;
+  const float* row = prod[0] + min(chain, Q * DS - 1) * LD;
+  constexpr int kBuf = Q * DS * LD;
+  float ra[kBlock], rb[kBlock];
+  auto read = [&](float (&r)[kBlock], int off) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < kBlock; k += 4) {
+      const float4 x = *reinterpret_cast<const float4*>(row + off + k);
+      r[k] = x.x;
+      r[k + 1] = x.y;
+      r[k + 2] = x.z;
+      r[k + 3] = x.w;
+    }
+  };
+  float acc = 0.0f;
+  flush_denorms();
+  auto add = [&](const float (&r)[kBlock]) __attribute__((always_inline)) {
+    tie(acc);
+#pragma unroll
+    for (int k = 0; k < kBlock; ++k) acc = __fadd_rn(acc, r[k]);
+    tie(acc);
+  };
+  lds_barrier();
+  read(ra, 0);
   for (int st = 0; st < NS; ++st) {
-    if (st + SLOTS - 1 < NS) issue(st + SLOTS - 1);
-    wait_stages_ahead<L, SLOTS - 1>(min(NS - 1 - st, SLOTS - 1));
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");  // the slot's reads stay after the barrier
-    if (active)
-      acc = pv_stage<VHALF, SR, ROWB>(acc, ring + SB * (st % SLOTS), d, sp + i * ldp + st * SR, min(SR, nk - st * SR),
-                                      vtest);
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's reads of the slot are done
-    __builtin_amdgcn_s_barrier();
+    read(rb, (st & 1) * kBuf + kBlock);
+    add(ra);
+    if (st + 1 < NS) {
+      lds_barrier();
+      read(ra, (~st & 1) * kBuf);
+    }
+    if (st * SK + kBlock < nk) add(rb);
   }
-  if (active) store_out(a.att[hg * G + i / M], (i % M) * a.ldatt, c * DS + d, a.out, chain_end(acc), a.out_scale);
+  keep_denorms();
+  tie(acc);
+  const int i = chain / DS, col = chain % DS;
+  if (i < Q) store_out(a.att[hg * G + i / M], (i % M) * a.ldatt, c * DS + col, a.out, chain_end(acc), a.out_scale);
 }
 
 // Columns over grid x (per / threads each), rows over grid y with a stride loop past 65535 rows.
@@ -1270,12 +1356,22 @@ int query_group(const AttnArgs& a) {
   return 1;
 }
 
+// AHEAD: V stages loaded ahead, no more than there are keys for (loads past them cost 4 queries over 104
+// keys 0.7 us).
+template <int Q, int AHEAD>
+void launch_split_pv(const AttnArgs& a, dim3 grid, hipStream_t s) {
+  static_assert(64 % kAttnSplitCols == 0, "every head size is a whole number of column blocks");
+  if (a.v_fp16) hipLaunchKernelGGL((attn_split_pv_kernel<true, Q, AHEAD>), grid, dim3(pv_threads(Q)), 0, s, a);
+  else hipLaunchKernelGGL((attn_split_pv_kernel<false, Q, AHEAD>), grid, dim3(pv_threads(Q)), 0, s, a);
+}
+
 template <int HD, int Q>
 void launch_split_q(const AttnArgs& a, dim3 gs, dim3 gp, hipStream_t s) {
   if (a.rope) hipLaunchKernelGGL((attn_split_scores_kernel<HD, Q, true>), gs, dim3(256), 0, s, a);
   else hipLaunchKernelGGL((attn_split_scores_kernel<HD, Q, false>), gs, dim3(256), 0, s, a);
-  if (a.v_fp16) hipLaunchKernelGGL((attn_split_pv_kernel<HD, true, Q>), gp, dim3(256), 0, s, a);
-  else hipLaunchKernelGGL((attn_split_pv_kernel<HD, false, Q>), gp, dim3(256), 0, s, a);
+  if (a.nk <= 2 * kPvStage) launch_split_pv<Q, 2>(a, gp, s);
+  else if (a.nk <= 4 * kPvStage) launch_split_pv<Q, 4>(a, gp, s);
+  else launch_split_pv<Q, 8>(a, gp, s);
 }
 
 template <int HD>
@@ -1360,13 +1456,13 @@ hipError_t launch_attention(const AttnArgs& in, hipStream_t s) {
   if (in.rope && !(split && in.M == 1 && in.hd % 32 == 0 && in.rope_key >= 0 && in.rope_key < in.nk))
     return hipErrorInvalidValue;  // split form only
   if (split) {
-    // the split form: scratch rows of the scores, 32 keys per scores workgroup (more past 512 keys,
-    // at most 16 chunks)
+    // the split form: scratch rows of the scores, 32 keys per scores workgroup (64 past 2048 keys: at 2048
+    // keys of 8 K / V heads 128 keys per workgroup, half the CUs' worth of them, cost 1.8 us a call)
     AttnArgs a = in;
     a.ld_scratch = (a.nk + 3) / 4 * 4;
     a.group = query_group(a);
     while (a.group > 1 && a.group * a.M * a.ld_scratch > kAttnSplitProbs) a.group /= 2;
-    a.keys_per_wg = 32 * ((a.nk + 511) / 512);
+    a.keys_per_wg = 32 * ((a.nk + 2047) / 2048);
     if (a.hd == 64) launch_split<64>(a, s);
     else if (a.hd == 128) launch_split<128>(a, s);
     else launch_split<256>(a, s);

@@ -77,7 +77,7 @@ CASES = [
     (6, 6, 128, 3, 60, False, OUT_INT8),     # 3 rows, no sharing
     (2, 1, 128, 4, 500, False, OUT_FP32),    # 4 rows: the group split back to single heads
     (2, 1, 64, 5, 30, False, OUT_FP32),      # 5 rows: one workgroup per head
-    (2, 1, 64, 1, 2000, True, OUT_FP32),     # 2016 keys: 128 keys per scores workgroup
+    (2, 1, 64, 1, 2000, True, OUT_FP32),     # 2016 keys: 63 scores workgroups per head
     (2, 2, 128, 1, 4070, False, OUT_FP32),   # 4080 keys, the most either form takes
     (4, 2, 128, 2, 3000, False, OUT_FP32),   # probabilities past the split form's LDS: one per head
     (3, 3, 64, 1, 0, False, OUT_FP32),       # the first position: one valid key of 16
@@ -98,6 +98,34 @@ def test_attention_matches_the_oracle(heads, kv_heads, hd, M, t0, v_fp16, out):
 ])
 def test_attention_with_values_the_flushes_change(heads, kv_heads, hd, M, t0, v_fp16):
     run_case(heads, kv_heads, hd, M, t0, v_fp16, OUT_FP32, specials=True)
+
+
+# the split form at the edges of its P V stages (64 keys, read in halves; 2, 4 or 8 stages ahead) and of the
+# scores' key chunks, 1 to 4 query rows per group (key counts are multiples of 4), with scores spread so far that probabilities underflow to
+# subnormal products and zeros; bit for bit, so no tolerance
+@pytest.mark.parametrize("nk,M,grp,v_fp16,specials", [
+    (4, 1, 1, False, False), (8, 2, 2, True, False), (28, 1, 2, False, True), (36, 3, 1, True, True),
+    (60, 1, 4, False, False), (64, 2, 1, False, True), (68, 1, 2, True, False), (124, 4, 1, False, True),
+    (128, 1, 4, True, True), (132, 1, 1, False, False), (252, 2, 2, False, True), (256, 1, 2, True, True),
+    (260, 3, 1, False, False), (508, 1, 2, True, True), (512, 4, 1, False, True), (516, 1, 4, False, True),
+    (580, 1, 2, False, True), (1028, 2, 1, True, True), (2052, 1, 1, False, True), (1092, 1, 2, True, False),
+])
+def test_split_attention_at_the_stage_edges(nk, M, grp, v_fp16, specials):
+    rng = np.random.default_rng(nk * 8 + M)
+    kv_heads, hd = 2, 64
+    heads = kv_heads * grp
+    q = rng.normal(0, 4.0, (M, heads * hd)).astype(f32)
+    kc = rng.normal(0, 1.5, (nk, kv_heads * hd)).astype(f32)
+    vv = rng.normal(0, 1, (nk, kv_heads * hd)).astype(f32)
+    if specials and nk >= 16:
+        plant_attention_specials(rng, q, kc, vv, kv_heads, hd, v_fp16)
+    vdev = vv.astype(np.float16).view(np.uint16) if v_fp16 else vv
+    vval = F.from_fp16_bits(vdev) if v_fp16 else vv
+    for causal_k in (0, max(1, nk - M + 1)):
+        got = ops.attention(q, kc, vdev, heads, kv_heads, causal_k=causal_k, v_fp16=v_fp16)
+        want, _, _ = oracle_attention(q, kc, vval, heads, kv_heads, hd, causal_k, OUT_FP32, None)
+        bad = np.argwhere(bits(got) != bits(want))
+        assert len(bad) == 0, f"causal_k={causal_k}: {len(bad)} differ, first at {tuple(bad[0])}"
 
 
 # prompt rows (16 query rows per workgroup): one row of a tile, whole and partial tiles, every head size
