@@ -943,6 +943,12 @@ hipError_t go_cpl(const W4Args& a, int cpl, hipStream_t s) {
 //     Past 2048 k, 16 waves per workgroup and the tile shape (4 rows; 8 rows; 8 rows and two
 //     weight tiles) with the largest grid of at most 256 workgroups: K = 6144, N = 1536: M = 8 /
 //     16 / 32: 6.6 / 7.8 / 11.6 us; K = 3072, N = 4096: M = 8 / 16: 6.0 / 8.5 us.
+//     The largest grids of both are bound by the waves in flight, which LDS (operands and terms sized for
+//     GMAX groups) limits: with GMAX for the row's groups instead of 16 or 48 (us, M x K x N): up to 4 groups
+//     8 weight tiles of one wave (1000 x 512 x 4096 91 -> 34; 4 tiles 38), up to 8 groups 4 tiles of two
+//     (512 x 1024 x 4096 61 -> 33; at 6 groups 163 -> 87), up to 12 groups 8 tiles of two waves (256 x 1536 x
+//     12288 97 -> 73; 4 tiles 74.5; with GMAX 16 they took 105), 18 to 24 groups two tiles of 8 waves (200 x
+//     3072 x 4096 85 -> 46; one tile of 16 waves 65).
 // The 8-row tiles with the two halves of the mantissa in the operand rows replaced tiles that
 // took them in separate MFMAs (4 rows per tile and masked operand rows): K = 1536, N = 12288:
 // M = 4 / 8 / 16 / 32: 6.3 / 9.1 / 12.5 / 22.1 -> 5.7 / 6.7 / 9.9 / 16.6 us.
@@ -967,11 +973,15 @@ hipError_t launch_gemv_w4a16(const W4Args& a, hipStream_t s) {
       if ((n16 + 1) / 2 * mb8 <= 256) return go_w4_mfma<8, 2, 16, 16>(a, s);
       if (n16 * mb8 <= 768) return go_w4_mfma<8, 1, 8, 16>(a, s);
       if ((n16 + 1) / 2 * mb8 <= 768) return go_w4_mfma<8, 2, 8, 16>(a, s);
+      if (G <= 4) return go_w4_mfma<8, 8, 8, 4>(a, s);
+      if (G <= 8) return go_w4_mfma<8, 4, 8, 8>(a, s);
+      if (G <= 12) return go_w4_mfma<8, 8, 16, 12>(a, s);
       return go_w4_mfma<8, 4, 8, 16>(a, s);
     }
     if (G <= 48) {
       if (n16 * mb4 <= 256) return go_w4_mfma<4, 1, 16, 48>(a, s);
       if (n16 * mb8 <= 256) return go_w4_mfma<8, 1, 16, 48>(a, s);
+      if (G <= 24) return go_w4_mfma<8, 2, 16, 24>(a, s);
       return go_w4_mfma<8, 2, 16, 48>(a, s);
     }
     return go_w4_mfma<4, 1, 16, 64>(a, s);

@@ -734,6 +734,17 @@ def test_c5_w4a16_gemma4(K, N, seed):
     assert same(host(y), want), mismatch(host(y), want)
 
 
+# the largest grids, by groups of a row: 2 to 4, to 8, to 12, to 16, 18 to 24 and more, with a partial last
+# weight tile and a partial last row tile
+@pytest.mark.parametrize("K,M,N", [(256, 203, 1040), (512, 203, 1040), (768, 203, 1040), (1024, 203, 1040),
+                                   (1280, 203, 1040), (1536, 203, 1040), (1792, 203, 1040), (2304, 67, 528),
+                                   (3072, 67, 528), (3328, 67, 528)])
+def test_w4a16_large_grids(K, M, N):
+    x, Wp, ws, _ = w4_inputs(K + M, M, N, K)
+    y, want = ops.gemm_w4(cuda(x), cuda(Wp), cuda(ws)), G.gemm_w4(x, Wp, ws)
+    assert same(host(y), want), mismatch(host(y), want)
+
+
 @pytest.mark.parametrize("K,N", [(1536, 12288), (6144, 1536)])
 @pytest.mark.parametrize("M", [2, 4, 5, 8])
 def test_w4a16_prefill_chunks(K, N, M):
