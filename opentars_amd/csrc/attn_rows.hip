@@ -102,7 +102,7 @@ __global__ __launch_bounds__(64 * (16 / RW) * (HD / 64), 2) void attn_rows_kerne
   const int h = nh % 8 == 0 ? (hb % 8) * (nh / 8) + hb / 8 : hb;
   const int m0 = (tiles - 1 - b / nh) * tr;
   const int rows = min(tr, a.M - m0), nk = a.nk;
-  const int limit = a.causal_k > 0 ? min(nk, a.causal_k + m0 + rows - 1) : nk;  // keys some row sees
+  const int limit = causal_valid(nk, a.causal_k, m0 + rows - 1);  // keys some row sees
   const bool last = h == nh - 1;
   const int score_keys = last && a.sc ? nk : limit;
   const v16f neg0 = splat(-0.0f);
@@ -216,7 +216,7 @@ __global__ __launch_bounds__(64 * (16 / RW) * (HD / 64), 2) void attn_rows_kerne
   for (int r = t >> 4; r < tr; r += 4 * nw) {
     float* s = sp + r * lds_row;
     const int m = m0 + min(r, rows - 1);
-    const int V = a.causal_k > 0 ? min(nk, a.causal_k + m) : nk;
+    const int V = causal_valid(nk, a.causal_k, m);
     // the lane's n elements l, l + 16, ... of the row, eight at a time (their chains of steps side by side)
     const int n = pad >> 4;
     auto each = [&](auto&& f) {

@@ -323,6 +323,12 @@ struct AttnNormRope {
   int rows_per_pos;
 };
 
+// Elements (keys) row m of a causal softmax over n sees: min(n, causal_k + m), or n when causal_k is 0. A
+// causal_k up to 2^31 - 1 is legal (no mask), so their sum is formed only when it is below n.
+__host__ __device__ __forceinline__ int causal_valid(int n, int causal_k, int m) {
+  return causal_k > 0 && m < n - causal_k ? causal_k + m : n;
+}
+
 struct AttnArgs {
   const float* q[kAttnMaxHeads];   // head h: query rows [M, hd] at ldq
   const float* k[kAttnMaxHeads];   // K rows [nk, hd] at ldk (fp32)

@@ -810,7 +810,7 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
     else if (nk <= 128) attn_scores<U, 8>(a, h, m, g, l, last, qv, sp);
     else attn_scores<U, KF>(a, h, m, g, l, last, qv, sp);
     // (2) causal softmax in place
-    const int V = a.causal_k > 0 ? min(nk, a.causal_k + m) : nk;
+    const int V = causal_valid(nk, a.causal_k, m);
     const int above1 = softmax_lds(sp, nk, V, last ? a.pr : nullptr, m * a.ldpr, red, &bcast);
     wait_vmcnt<0>();  // the first V stages have landed; nothing else outstanding before the ring's counts
     // V elements need their own test only when fp32 and some probability is above 1 or NaN: with
@@ -1037,7 +1037,7 @@ __device__ __forceinline__ void softmax_rows_lds(float* sp, int ldp, int M, int 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int i = wave / W, t = static_cast<int>(threadIdx.x) - i * T;
   const bool mine = i < Q;  // (a last wave can be left over)
-  const int V = causal_k > 0 ? min(nk, causal_k + i % M) : nk;
+  const int V = causal_valid(nk, causal_k, i % M);
   float* const s = sp + i * ldp;
   __syncthreads();  // the rows are complete
   // the maximum key of the row's valid keys, a NaN counting as 0xFFFFFFFF (above every other key:

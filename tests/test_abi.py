@@ -237,6 +237,24 @@ def test_overlap_of_strided_rows_matches_a_walk_over_the_rows():
     assert len(seen) == 4
 
 
+def test_causal_valid_counts_at_the_ends_of_32_bits(tmp_path):
+    """causal_valid (the keys a row of every causal softmax kernel sees), compiled for the host, against
+    min(n, causal_k + m) in Python's integers: causal_k near 2^31, rows near 2^31."""
+    from opentars_amd import build
+    top = 2 ** 31 - 1
+    cases = [(n, k, m) for n in (1, 2, 17, 4080, top) for k in (0, 1, 16, 4079, 4080, top - 4080, top - 39, top - 1, top)
+             for m in (0, 1, 15, 39, 4080, top - 4080, top - 1)]
+    src = tmp_path / "valid.hip"
+    src.write_text('#include <cstdio>\n#include "kernels.h"\nint main() {\n  int n, k, m;\n'
+                   '  while (std::scanf("%d %d %d", &n, &k, &m) == 3) std::printf("%d\\n", tars::causal_valid(n, k, m));\n}\n')
+    exe = tmp_path / "valid"
+    subprocess.run([build.hipcc(), "--offload-arch=gfx950", "--offload-host-only", "-std=c++17", "-O1", "-w", "-I", str(build.CSRC),
+                    str(src), "-o", str(exe)], check=True, capture_output=True)
+    out = subprocess.run([str(exe)], input="\n".join("%d %d %d" % c for c in cases), capture_output=True, text=True, check=True)
+    got = [int(x) for x in out.stdout.split()]
+    assert got == [min(n, k + m) if k > 0 else n for n, k, m in cases]
+
+
 def test_fused_validation():
     lib = _lib.lib()
     W8 = _lib.W8A8Out

@@ -171,6 +171,21 @@ def test_masked_keys_of_prompt_rows_that_change_a_sum(v_fp16):
     assert np.array_equal(bits(got), bits(want))
 
 
+@pytest.mark.parametrize("M,nk,hd", [(2, 48, 128), (4, 100, 64), (5, 48, 128), (40, 100, 64), (33, 64, 256)])
+@pytest.mark.parametrize("causal_k", [2 ** 31 - 1, 2 ** 31 - 3])
+def test_causal_k_near_the_largest_int_is_no_mask(M, nk, hd, causal_k):
+    """min(nk, causal_k + m) is nk for every row, whatever causal_k + m is in 32 bits: the same as causal_k = 0,
+    the scores and probabilities with it. The split form (2 and 4 rows) and prompt rows."""
+    rng = np.random.default_rng(M)
+    q, kc, vv = (rng.normal(0, 0.5, s).astype(f32) for s in ((M, 2 * hd), (nk, hd), (nk, hd)))
+    sc, pr = (torch.full((M, nk), float("nan"), device="cuda") for _ in range(2))
+    got = ops.attention(q, kc, vv, 2, 1, causal_k=causal_k, sc=sc, pr=pr)
+    want, s_last, p_last = oracle_attention(q, kc, vv, 2, 1, hd, 0, OUT_FP32, None)
+    assert np.array_equal(bits(got), bits(want))
+    assert np.array_equal(bits(sc.cpu().numpy()), bits(s_last))
+    assert np.array_equal(bits(pr.cpu().numpy()), bits(p_last))
+
+
 def test_attention_twice_in_a_row_and_without_the_shared_rows():
     """Two calls on one stream share the device scratch: the second (fewer keys, other heads)
     must not see the first's scores; sc / pr left out."""
