@@ -165,7 +165,7 @@ __global__ __launch_bounds__(kRowThreads) void row_lds_kernel(RowArgs a) {
     }
   }
   if (a.fn == ROWFN_SOFTMAX) {
-    const int V = a.valid ? min(max(a.valid[m], 1), N) : (a.causal_k > 0 ? min(N, a.causal_k + m) : N);
+    const int V = a.valid ? min(max(a.valid[m], 1), N) : causal_valid(N, a.causal_k, m);
     __syncthreads();
     uint32_t key = 0;
     int nan = 0;
@@ -304,7 +304,7 @@ __global__ __launch_bounds__(kRowThreads) void row_kernel(RowArgs a) {
   const int N = a.N;
   const int64_t yrow = m * a.ldy;
   if (a.fn == ROWFN_SOFTMAX) {
-    const int V = a.valid ? min(max(a.valid[m], 1), N) : (a.causal_k > 0 ? min(N, a.causal_k + m) : N);
+    const int V = a.valid ? min(max(a.valid[m], 1), N) : causal_valid(N, a.causal_k, m);
     uint32_t key = 0;
     int nan = 0;
     for_lane(x, l, V, [&](int, float xv) {

@@ -68,6 +68,15 @@ def test_softmax_causal_reference_vectors(name):
     assert same(got, VEC[name + "_y"]), mismatch(got, VEC[name + "_y"])
 
 
+@pytest.mark.parametrize("M,N", [(5, 96), (3, 13000)])
+@pytest.mark.parametrize("k", [2 ** 31 - 1, 2 ** 31 - 2])
+def test_softmax_causal_k_near_the_largest_int_is_no_mask(M, N, k):
+    """min(N, k + m) is N for every row, whatever k + m is in 32 bits (rows in LDS and longer rows)."""
+    x = rows_with_specials(M + N, M, N, scale=4.0)
+    got, want = ops.softmax_rows(x, causal_k=k), R.softmax_rows(x)
+    assert same(got, want), mismatch(got, want)
+
+
 @pytest.mark.parametrize("out", OUTS)
 @pytest.mark.parametrize("M,N,k", [(1, 16, 0), (7, 80, 0), (16, 250, 0), (33, 512, 0), (16, 256, 5), (9, 96, 90),
                                    (3, 4096, 0), (2, 12288, 0), (2, 13000, 7000)])
