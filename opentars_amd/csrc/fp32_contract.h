@@ -217,6 +217,24 @@ __device__ __forceinline__ float act_fn(float x, int act) {
   }
 }
 
+// act_fn of four values: one branch on the code, and the four chains of an activation side by side.
+__device__ __forceinline__ void act_fn4(float (&y)[4], int act) {
+  auto each = [&](auto fn) __attribute__((always_inline)) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) y[v] = fn(ftz(y[v]));
+  };
+  switch (act) {
+    case 0: each([](float x) { return x; }); break;
+    case 1: each([](float x) { return relu_plain(x); }); break;
+    case 2: each([](float x) { const float r = relu_plain(x); return r > 6.0f ? 6.0f : r; }); break;
+    case 3: each([](float x) { return gelu_f(x); }); break;
+    case 4: each([](float x) { return silu_f(x); }); break;
+    case 5: each([](float x) { return sigmoid_f(x); }); break;
+    case 6: each([](float x) { return softplus_f(x); }); break;
+    default: each([](float x) { return exp_f(x); });
+  }
+}
+
 // numerics.py:282-286: rint(fmul(x, inv)) ties-to-even, NaN -> 0, clamp to [-127, 127]
 __device__ __forceinline__ int8_t q8(float x, float inv) {
   float y = fmul(x, inv);

@@ -523,7 +523,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void mfma_wide_kernel(const int8_t
   // rows of the output tile staged through LDS at a time
   constexpr int OM = BM * TP * 4 <= S * SLOT ? BM : BM / 2;
   static_assert(BLK % NW == 0 && L * (S - 1) < 64 && S >= 3 && OM * TP * 4 <= S * SLOT && (OM == BM || WM % 2 == 0), "wide tile");
-  __shared__ __align__(16) int8_t lds[S * SLOT];
+  __shared__ __align__(16) int8_t lds[S * SLOT + (KSPLIT ? 0 : 4 * BM)];  // the ring (later the sums), the rows' scales
+  float* const row_scales = reinterpret_cast<float*>(lds + S * SLOT);
   const v4i zero = {0, 0, 0, 0};
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -547,6 +548,23 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void mfma_wide_kernel(const int8_t
     }
 #pragma unroll
     for (int i = 0; i < TI; ++i) sr[i] = *(srow ? srow + min(m0 + (wm * TI + i) * 16 + li, M - 1) : scol);
+    issue_fence();
+  }
+
+  // The epilogue's operands, loaded before the stages so that no tile ends on their latency: its four columns'
+  // scales and biases, and one row's scale per thread, which goes through LDS.
+  constexpr int Q = BN / 4, RS = NT / Q;
+  static_assert(NT % Q == 0 && OM % RS == 0, "a thread keeps its columns");
+  const int cq = static_cast<int>(threadIdx.x) % Q, n = n0 + 4 * cq, nc = min(n, N - 4);
+  float4 c4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), b4 = c4;
+  if constexpr (!KSPLIT) {
+    if (SIMPLE || !tl.scol_per_tensor) c4 = *reinterpret_cast<const float4*>(scol + nc);
+    else c4 = make_float4(scol[0], scol[0], scol[0], scol[0]);
+    if (!SIMPLE && tl.bias) b4 = *reinterpret_cast<const float4*>(tl.bias + nc);
+  }
+  float srv = 0.0f;
+  if constexpr (!KSPLIT) {
+    srv = *(srow ? srow + min(m0 + min(static_cast<int>(threadIdx.x), BM - 1), M - 1) : scol);
     issue_fence();
   }
 
@@ -648,18 +666,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void mfma_wide_kernel(const int8_t
     }
   }
   // The sums (a K split: the outputs) go through LDS, OM rows of the tile at a time; there a thread owns
-  // four columns of every NT / (BN / 4)-th row, so it loads its column scales and biases once, and a row's
-  // consecutive 16-byte pieces are stored by consecutive threads.
+  // four columns of every NT / (BN / 4)-th row, so a row's consecutive 16-byte pieces are stored by consecutive threads.
   int32_t* tile = reinterpret_cast<int32_t*>(lds);
-  constexpr int Q = BN / 4, RS = NT / Q;
-  static_assert(NT % Q == 0 && OM % RS == 0, "a thread keeps its columns");
-  const int cq = static_cast<int>(threadIdx.x) % Q, n = n0 + 4 * cq, nc = min(n, N - 4);
-  float4 c4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), b4 = c4;
-  if constexpr (!KSPLIT) {
-    if (SIMPLE || !tl.scol_per_tensor) c4 = *reinterpret_cast<const float4*>(scol + nc);
-    else c4 = make_float4(scol[0], scol[0], scol[0], scol[0]);
-    if (!SIMPLE && tl.bias) b4 = *reinterpret_cast<const float4*>(tl.bias + nc);
-  }
+  if (!KSPLIT && threadIdx.x < BM) row_scales[threadIdx.x] = srv;
 #pragma unroll
   for (int h = 0; h < BM / OM; ++h) {
     __syncthreads();  // the stages (or the rows before) have been read
@@ -677,11 +686,16 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void mfma_wide_kernel(const int8_t
         }
     }
     __syncthreads();
-#pragma unroll 4
+    // the general epilogue one row (four outputs) at a time, with one branch on the activation. Four rows unrolled
+    // with a branch per output (sixteen copies of every activation) and the row scales loaded here cost more
+    // instruction fetch and latency than the overlap gave: M = 64, K = 272, N = 1040, SILU, INT8 8.0 -> 6.6 us,
+    // M = 2048, K = N = 4096 with INT8 output 54 -> 49 us (fp32, no activation 43.8 -> 41.9)
+    constexpr int kRows = SIMPLE || KSPLIT ? 4 : 1;
+#pragma unroll kRows
     for (int r = static_cast<int>(threadIdx.x) / Q; r < OM; r += RS) {
       const int m = m0 + h * OM + r;
       const v4i o = *reinterpret_cast<const v4i*>(tile + r * TP + 4 * cq);
-      const float srm = KSPLIT ? 0.0f : *(srow ? srow + min(m, M - 1) : scol);
+      const float srm = KSPLIT ? 0.0f : row_scales[h * OM + r];
       float y[4];
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
@@ -697,9 +711,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void mfma_wide_kernel(const int8_t
           if (srow) y[v] = fmul(y[v], srm);
           y[v] = fmul(y[v], sv);
           if (tl.bias) y[v] = fadd(y[v], bv);
-          y[v] = act_fn(y[v], tl.act);
         }
       }
+      if constexpr (!SIMPLE && !KSPLIT) act_fn4(y, tl.act);
       if (m < M && n < N) {
         if constexpr (SIMPLE || KSPLIT) {
           *reinterpret_cast<float4*>(static_cast<char*>(Y) + static_cast<int64_t>(m) * ldy + 4 * n) =

@@ -636,6 +636,26 @@ def test_wide_tiles(M, N, K, act, out, qm):
     assert same(host(y), want), mismatch(host(y), want)
 
 
+@pytest.mark.parametrize("act", range(8))
+@pytest.mark.parametrize("out", [OUT_FP32, OUT_BF16, OUT_INT8])
+def test_wide_tiles_with_every_activation(act, out):
+    """The general epilogue of the wide tiles (four values of a row at a time) with every activation and output
+    format, on column scales that make infinite, NaN, huge and subnormal products."""
+    M, N, K = 97, 2064, 1152
+    rng = np.random.default_rng(act * 3 + out)
+    A = rng.integers(-128, 128, (M, K), dtype=np.int8)
+    W = rng.integers(-128, 128, (N, K), dtype=np.int8)
+    sc = rng.uniform(1e-5, 3e-4, N).astype(f32)
+    sc[rng.choice(N, 12, replace=False)] = np.array([np.inf, -np.inf, np.nan, 1e38, -1e38, 1e-40, -1e-40, 1e-44, 0.0, -0.0,
+                                                     2e-38, 1e30], f32)
+    srow = rng.uniform(0.1, 2.0, M).astype(f32)
+    b = rng.normal(0, 2, N).astype(f32)
+    osc = f32(5.0) if out == OUT_INT8 else None
+    y = ops.gemm_rowcol(cuda(A), cuda(srow), cuda(W), cuda(sc), cuda(b), act=act, out=out, out_scale=osc)
+    want = G.gemm_rowcol(A, srow, W, sc, b, act=act, out=out, out_scale=osc)
+    assert same(host(y), want), mismatch(host(y), want)
+
+
 @pytest.mark.parametrize("M,N,blocks", [(100, 12304, [128, 144, 16]), (200, 6160, [512, 256]), (130, 4112, [48, 1040]),
                                         (40, 1040, [272, 128])])
 def test_ksplit_wide_tiles(M, N, blocks):
