@@ -1066,7 +1066,7 @@ hipError_t go_chunk(const MfmaArgs& a, hipStream_t s) {
 //  * 64 x 128 wide tiles from 192 of them: M = 1024, K = 1024, N = 3072 14.9 -> 10.7 us, M = 777, K = 4096, N = 4096
 //    43 -> 24 us, M = 512, K = 1152, N = 6912 35.6 -> 12.0 us (32 x 32 direct tiles before). With GELU and the
 //    activations after it the epilogue weighs as much as the sums, and below 512 tiles a CU with two of them
-//    holds the others up: M = 333, K = 1152, N = 6912 28 us, 22 us on 64 x 64 wide tiles;
+//    holds the others up: M = 333, K = 1152, N = 6912 26.6 us, 20.8 us on 64 x 64 wide tiles;
 //  * whole 256-byte stages and at most 512 32 x 32 tiles: the 32 x 32 ring with 256-byte stages (M = 512,
 //    K = 3072, N = 1024 8.2 us, 32 x 64 wide 8.6; at 640 tiles, M = 130, K = N = 4096, 19.6 against 12.0);
 //  * 64 x 64 wide tiles from 192 of them (M = 777, K = 3072, N = 1024 16.9 -> 10.4 us), else 32 x 64 wide tiles
@@ -1074,6 +1074,21 @@ hipError_t go_chunk(const MfmaArgs& a, hipStream_t s) {
 //  * the direct kernel's 32 x 32 tiles with 4 waves over K for few tiles of a long K that is not whole
 //    stages (M = 20, K = 2064, N = 2048 6.2 us, 32 x 64 wide 6.8) and for row strides the LDS kernels' 32-bit
 //    offsets do not cover. A K split runs the same rules without the 128 x 256 tiles.
+// A general epilogue (anything but fp32 output with row and column scales alone) costs a wave its instructions per
+// output: a 32 x 64 tile gives each of its four waves twice the outputs of a 32 x 32 tile, while SIMDs of a small grid
+// idle. "Chains" are GELU, SILU, sigmoid and softplus, 70 to 120 dependent instructions each. Measured over 1582
+// shapes (M = 17 - 2048, K = 128 - 6912, N = 512 - 12288) with up to seven epilogues each, the lines where the two sides
+// were equal:
+//  * K below 640 and not whole 256-byte stages: the direct 32 x 32 tiles up to 768 of them, with chains up to 1536, with
+//    softplus at any number (M = 64, K = 272, N = 1040, GELU 5.8 us, 32 x 64 wide 7.5; M = 900, K = 272, N = 6912, softplus
+//    45 us, 128 x 256 wide 60; at K = 640 the two are equal at 256 tiles);
+//  * no 128 x 256 tiles with chains below K = 1024, where a CU's one tile ends in 64 outputs per thread with nothing
+//    beside it (M = 900, K = 272, N = 6912, GELU 46 us, 64 x 128 wide 38);
+//  * whole 256-byte stages: the 32 x 32 ring up to 768 tiles (M = 130, K = 1024, N = 4096, INT8 output 6.2 us, 64 x 64 wide
+//    6.7, GELU 8.4 and 10.1), with chains and K up to 2048 again from 257 64 x 64 tiles, the second round of which nearly
+//    every CU would wait for, to 1536 32 x 32 tiles (M = 333, K = 1024, N = 3072, GELU 12.7 us, 64 x 64 wide 14.0);
+//  * chains on at most 256 32 x 32 tiles of other K: the direct kernel (M = 100, K = 2064, N = 2048, softplus 10.6 us, 32 x 64
+//    wide 12.3).
 bool whole_stages(const MfmaArgs& a, int ks) {
   for (int i = 0; i < a.nseg; ++i)
     if (a.seg[i].K % ks) return false;
@@ -1096,10 +1111,16 @@ hipError_t run(const MfmaArgs& a, hipStream_t s) {
   // the LDS kernels take 32-bit offsets inside a tile's rows; the direct kernel any strides
   if (a.lda >= (1 << 24) || a.ldy > INT32_MAX) return go_direct<2, 2, 4, 1>(a, s);
   const bool whole = whole_stages(a, 256);
+  int longest = 0;
+  for (int i = 0; i < a.nseg; ++i) longest = a.seg[i].K > longest ? a.seg[i].K : longest;
   const int64_t tw = tiles(a, 128, 256), tc = tiles(a, 64, 128), t48 = tiles(a, 64, 48), t64 = tiles(a, 64, 64),
                 t32 = tiles(a, 32, 32);
   const int64_t rounds = (tw + 255) / 256 * 256;  // 128 x 256 tiles that whole rounds would hold
-  if (a.nseg == 1 && tw >= 192 && (5 * tw >= 4 * rounds || (a.seg[0].K >= 2048 && 4 * tw >= 3 * rounds)))
+  const bool simple = a.nseg > 1 || simple_epilogue(a.epi);
+  const bool chains = a.epi.act >= 3 && a.epi.act <= 6, softplus = a.epi.act == 6;
+  if (!whole && !simple && longest < 640 && (softplus || t32 <= (chains ? 1536 : 768))) return go_direct<2, 2, 4, 1>(a, s);
+  if (a.nseg == 1 && tw >= 192 && !(chains && longest < 1024) &&
+      (5 * tw >= 4 * rounds || (a.seg[0].K >= 2048 && 4 * tw >= 3 * rounds)))
     return go_wide<128, 256, 2, 4, 3>(a, s);
   if (whole && t48 >= 192 && t48 <= 256) {
     if (a.nseg == 1 && a.seg[0].K <= 1280) {
@@ -1114,11 +1135,12 @@ hipError_t run(const MfmaArgs& a, hipStream_t s) {
     return go_tile<64, 48, 4, 1, 256, 3>(a, s);
   }
   if (t32 <= 256 && whole_stages(a, 1024)) return go_tile<32, 32, 2, 2, 512, 3>(a, s);
+  if (whole && !simple && (t32 <= 768 || (chains && t64 > 256 && t32 <= 1536 && longest <= 2048)))
+    return go_tile<32, 32, 2, 2, 256, 3>(a, s);
+  if (!whole && chains && t32 <= 256) return go_direct<2, 2, 4, 1>(a, s);
   if (tc >= 192 && (tc >= 512 || a.epi.act < 3)) return go_wide<64, 128, 2, 4, 3>(a, s);
   if (whole && t32 <= 512) return go_tile<32, 32, 2, 2, 256, 3>(a, s);
   if (t64 >= 192) return go_wide<64, 64, 2, 4, 4>(a, s);
-  int longest = 0;
-  for (int i = 0; i < a.nseg; ++i) longest = a.seg[i].K > longest ? a.seg[i].K : longest;
   if (tiles(a, 32, 64) < 96 && longest > 1280) return go_direct<2, 2, 4, 1>(a, s);
   return go_wide<32, 64, 2, 2, 4>(a, s);
 }

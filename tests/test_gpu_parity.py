@@ -12,7 +12,7 @@ import torch
 from oracle import golden as G
 from oracle import numerics as F
 from opentars_amd import ops
-from opentars_amd.contract import (ACT_GELU, ACT_NONE, ACT_RELU, ACT_SILU, ACT_SOFTPLUS, OUT_BF16, OUT_FP32,
+from opentars_amd.contract import (ACT_EXP, ACT_GELU, ACT_NONE, ACT_RELU, ACT_SIGMOID, ACT_SILU, ACT_SOFTPLUS, OUT_BF16, OUT_FP32,
                                    OUT_INT8)
 
 pytestmark = pytest.mark.gpu
@@ -652,6 +652,33 @@ def test_wide_tiles_with_every_activation(act, out):
     b = rng.normal(0, 2, N).astype(f32)
     osc = f32(5.0) if out == OUT_INT8 else None
     y = ops.gemm_rowcol(cuda(A), cuda(srow), cuda(W), cuda(sc), cuda(b), act=act, out=out, out_scale=osc)
+    want = G.gemm_rowcol(A, srow, W, sc, b, act=act, out=out, out_scale=osc)
+    assert same(host(y), want), mismatch(host(y), want)
+
+
+# prompt rows by epilogue, ragged, on each side of the rules for general epilogues: 128 x 256 wide tiles with a light
+# activation; 64 x 64 and 32 x 64 wide tiles with K shorter than a stage; 32 x 64 wide tiles with chains; the direct
+# tiles at short K (chains past 768 tiles, softplus past 1536) and with chains at any K; the 32 x 32 ring up to 768
+# tiles and, with chains, past 1024
+@pytest.mark.parametrize("M,N,K,act,out,qm,bias", [
+    (257, 18688, 256, ACT_EXP, OUT_BF16, "channel", True),
+    (161, 4432, 48, ACT_EXP, OUT_FP32, "rowcol", True), (33, 1040, 112, ACT_NONE, OUT_FP32, "rowcol", False),
+    (97, 4112, 656, ACT_SILU, OUT_INT8, "rowcol", True),
+    (130, 1040, 272, ACT_SOFTPLUS, OUT_INT8, "rowcol", True), (200, 4112, 528, ACT_GELU, OUT_FP32, "rowcol", False),
+    (260, 5648, 16, ACT_SOFTPLUS, OUT_BF16, "tensor", True), (65, 1040, 1040, ACT_SIGMOID, OUT_FP32, "channel", True),
+    (130, 4112, 768, ACT_NONE, OUT_INT8, "rowcol", False), (333, 3088, 512, ACT_GELU, OUT_BF16, "rowcol", True),
+])
+def test_prompt_rows_by_epilogue(M, N, K, act, out, qm, bias):
+    rng = np.random.default_rng(M * 3 + K)
+    A = rng.integers(-128, 128, (M, K), dtype=np.int8)
+    W = rng.integers(-128, 128, (N, K), dtype=np.int8)
+    sc = rng.uniform(1e-4, 3e-2, N).astype(f32)
+    sc = sc[:1] if qm == "tensor" else sc
+    srow = rng.uniform(0.1, 2.0, M).astype(f32) if qm == "rowcol" else None
+    b = rng.normal(0, 2, N).astype(f32) if bias else None
+    osc = f32(5.0) if out == OUT_INT8 else None
+    y = ops.gemm_rowcol(cuda(A), None if srow is None else cuda(srow), cuda(W), cuda(sc), None if b is None else cuda(b),
+                        act=act, out=out, out_scale=osc)
     want = G.gemm_rowcol(A, srow, W, sc, b, act=act, out=out, out_scale=osc)
     assert same(host(y), want), mismatch(host(y), want)
 
