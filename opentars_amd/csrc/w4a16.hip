@@ -975,7 +975,8 @@ hipError_t launch_gemv_w4a16(const W4Args& a, hipStream_t s) {
       if ((n16 + 1) / 2 * mb8 <= 768) return go_w4_mfma<8, 2, 8, 16>(a, s);
       if (G <= 4) return go_w4_mfma<8, 8, 8, 4>(a, s);
       if (G <= 8) return go_w4_mfma<8, 4, 8, 8>(a, s);
-      if (G <= 12) return go_w4_mfma<8, 8, 16, 12>(a, s);
+      const int64_t wide = (n16 + 7) / 8 * mb8;  // workgroups of 8 weight tiles
+      if (G <= 12 && (wide <= 256 || wide > 320)) return go_w4_mfma<8, 8, 16, 12>(a, s);
       return go_w4_mfma<8, 4, 8, 16>(a, s);
     }
     if (G <= 48) {
