@@ -1,11 +1,14 @@
 """tars_attention (opentars_amd.ops.attention) against the oracle's three ops per head, bit for bit:
 fdot_nt of the head's q rows with its K head's rows, the causal softmax, fdot_nn with the V rows
 (the reference's lowering, tars_mini/llm.py:736-746), and the last head's scores and
-probabilities in the shared rows. The shapes cover both forms of the kernel: the split form (up to
-4 query rows per K / V head group: Qwen3 decode with 2 query heads per K / V head, Gemma-style 4,
-2- to 4-row chunks, long contexts) and one workgroup per head (5 rows, or probabilities past the
-split form's LDS). Needs a gfx950 GPU."""
+probabilities in the shared rows. The shapes cover the three forms: the split form (up to 4 query
+rows per K / V head group: Qwen3 decode with 2 query heads per K / V head, Gemma-style 4, 2- to 4-row
+chunks, long contexts), prompt rows (16 query rows of a head per workgroup: 5 rows and more, or
+probabilities past the split form's LDS) and one workgroup per head (one row of a stream without a
+scratch, V rows 128 MiB or more apart). Needs a gfx950 GPU."""
 from __future__ import annotations
+
+import ctypes
 
 import numpy as np
 import pytest
@@ -16,6 +19,7 @@ from oracle import golden as G
 from oracle import numerics as F
 from oracle import rowops as R
 from opentars_amd import ops
+from opentars_amd.build import LIB
 from opentars_amd.contract import OUT_BF16, OUT_FP32, OUT_INT8
 
 pytestmark = pytest.mark.gpu
@@ -76,10 +80,10 @@ CASES = [
     (8, 4, 64, 2, 100, False, OUT_BF16),     # a 2-row chunk: 4 query rows per group
     (6, 6, 128, 3, 60, False, OUT_INT8),     # 3 rows, no sharing
     (2, 1, 128, 4, 500, False, OUT_FP32),    # 4 rows: the group split back to single heads
-    (2, 1, 64, 5, 30, False, OUT_FP32),      # 5 rows: one workgroup per head
+    (2, 1, 64, 5, 30, False, OUT_FP32),      # 5 rows: the prompt-row kernel
     (2, 1, 64, 1, 2000, True, OUT_FP32),     # 2016 keys: 63 scores workgroups per head
-    (2, 2, 128, 1, 4070, False, OUT_FP32),   # 4080 keys, the most either form takes
-    (4, 2, 128, 2, 3000, False, OUT_FP32),   # probabilities past the split form's LDS: one per head
+    (2, 2, 128, 1, 4070, False, OUT_FP32),   # 4080 keys, the most any form takes
+    (4, 2, 128, 2, 3000, False, OUT_FP32),   # probabilities past the split form's LDS: the prompt-row kernel
     (3, 3, 64, 1, 0, False, OUT_FP32),       # the first position: one valid key of 16
 ]
 
@@ -219,6 +223,60 @@ def test_attention_on_two_streams_at_once():
     for j in (0, 1):
         for rep, att in enumerate(outs[j]):
             assert np.array_equal(bits(att.cpu().numpy()), bits(data[j][1])), f"stream {j}, call {rep}"
+
+
+def graph_nodes(g: torch.cuda.CUDAGraph) -> int:
+    n = ctypes.c_size_t(0)
+    assert ctypes.CDLL(str(LIB)).hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value
+
+
+# without a scratch: one workgroup per head for one row (up to 64 keys, up to 128, and more take different numbers of
+# keys at a time), the prompt-row kernel for 3
+@pytest.mark.parametrize("heads,kv_heads,hd,M,t0,v_fp16,specials", [
+    (4, 2, 128, 1, 40, False, True), (2, 1, 64, 1, 100, True, True), (2, 2, 256, 1, 60, False, False),
+    (8, 1, 64, 1, 300, False, True), (2, 1, 256, 1, 250, True, True), (2, 1, 128, 1, 2100, True, False),
+    (2, 1, 128, 1, 4070, False, False), (4, 2, 128, 3, 60, False, True),
+])
+def test_first_attention_of_a_stream_inside_a_graph_capture(heads, kv_heads, hd, M, t0, v_fp16, specials):
+    """A stream whose first attention call is captured gets no scratch (nothing is allocated under capture): one
+    kernel instead of the split form's two. Every replay equals the oracle, with eager calls between them."""
+    q, kc, vdev, vval, nk = layer(900 + t0 + hd, heads, kv_heads, hd, M, t0, v_fp16, specials)
+    want, s_last, p_last = oracle_attention(q, kc, vval, heads, kv_heads, hd, t0 + 1, OUT_FP32, None)
+    dq, dk, dv = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (q, kc, vdev.view(np.int16) if v_fp16 else vdev))
+    att = torch.empty((M, heads * hd), device="cuda")
+    sc, pr = torch.empty((M, nk), device="cuda"), torch.empty((M, nk), device="cuda")
+    hip, handle = ctypes.CDLL(str(LIB)), ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(handle)) == 0   # torch's own streams come from a pool: another test's, perhaps
+    stream = torch.cuda.ExternalStream(handle.value)
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g, stream=stream):
+        ops.attention(dq, dk, dv, heads, kv_heads, causal_k=t0 + 1, v_fp16=v_fp16, att=att, sc=sc, pr=pr)
+    assert graph_nodes(g) == 1
+    for rep in range(3):
+        for t in (att, sc, pr):
+            t.fill_(float("nan"))
+        eager = ops.attention(dq, dk, dv, heads, kv_heads, causal_k=t0 + 1, v_fp16=v_fp16)
+        g.replay()
+        torch.cuda.synchronize()
+        for t, w in ((att, want), (sc, s_last), (pr, p_last), (eager, want)):
+            assert np.array_equal(bits(t.cpu().numpy()), bits(w)), f"replay {rep}"
+    del g
+    assert hip.hipStreamDestroy(handle) == 0
+
+
+def test_rows_of_v_128_mib_apart():
+    """V row strides past the prompt-row kernel's 32-bit offsets: one workgroup per head, its rows one after another."""
+    heads, hd, M, nk, causal_k = 2, 64, 6, 6, 2
+    rng = np.random.default_rng(8)
+    q, kc, vv = (rng.normal(0, 0.5, s).astype(f32) for s in ((M, heads * hd), (nk, hd), (nk, hd)))
+    v = torch.empty(((nk - 1) << 25) + hd, device="cuda").as_strided((nk, hd), (1 << 25, 1))
+    v.copy_(torch.from_numpy(vv))
+    sc, pr = torch.empty((M, nk + 2), device="cuda")[:, :nk], torch.empty((M, nk + 2), device="cuda")[:, :nk]
+    att = ops.attention(torch.from_numpy(q).cuda(), torch.from_numpy(kc).cuda(), v, heads, 1, causal_k=causal_k, sc=sc, pr=pr)
+    want, s_last, p_last = oracle_attention(q, kc, vv, heads, 1, hd, causal_k, OUT_FP32, None)
+    for t, w in ((att, want), (sc, s_last), (pr, p_last)):
+        assert np.array_equal(bits(t.cpu().numpy()), bits(w))
 
 
 def test_attention_refusals():
