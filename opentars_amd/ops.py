@@ -471,10 +471,10 @@ def attention(q, kcache, vcache, heads: int, kv_heads: int, causal_k: int = 0, v
     ve, oe, grp = (2 if v_fp16 else 4), ESIZE[out], heads // kv_heads
     ptrs = ctypes.c_void_p * heads
     q0, k0, v0, a0 = qt.data_ptr(), kt.data_ptr(), vt.data_ptr(), att.data_ptr()
-    qp = ptrs(*range(q0, q0 + 4 * hd * heads, 4 * hd))
+    qp = ptrs(*range(q0, q0 + 4 * hd * heads, 4 * hd or 1))   # zero-wide heads: NULL, the library's error
     kp = ptrs(*[k0 + 4 * hd * (h // grp) for h in range(heads)])
     vp = ptrs(*[v0 + ve * hd * (h // grp) for h in range(heads)])
-    ap = ptrs(*range(a0, a0 + oe * hd * heads, oe * hd))
+    ap = ptrs(*range(a0, a0 + oe * hd * heads, oe * hd or 1))
     osb = _f32_bits(out_scale) if out == OUT_INT8 else 0
     _check(_lib.lib().tars_attention(qp, _ld(qt), kp, _ld(kt), vp, _ld(vt), int(v_fp16), ap, _ld(att), out, osb,
                                      _ptr(sc), 0 if sc is None else _ld(sc), _ptr(pr), 0 if pr is None else _ld(pr),

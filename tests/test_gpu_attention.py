@@ -289,3 +289,9 @@ def test_attention_refusals():
     with pytest.raises(ops.TarsError):
         ops.attention(torch.zeros((1, 96), device="cuda"), torch.zeros((32, 48), device="cuda"),
                       torch.zeros((32, 48), device="cuda"), 2, 1)   # head size 48
+
+
+def test_zero_wide_heads_are_refused_by_the_library():
+    q, kc = torch.zeros((1, 0), device="cuda"), torch.zeros((32, 0), device="cuda")
+    with pytest.raises(ops.TarsError):
+        ops.attention(q, kc, kc, 2, 1)
