@@ -57,19 +57,6 @@ constexpr int kKeys = 16;  // keys per block of P V
 constexpr int kAhead = 2;  // blocks of V rows in flight
 constexpr size_t kLds = 163840;  // LDS of a CU
 
-// fp32 subnormals kept / flushed (MODE bits 4-5) from here on. The values an instruction of a region
-// takes or gives pass through tie() inside it: the compiler keeps volatile statements in order, so
-// it cannot move the instruction out of its region. Between kernels' phases the mode is "keep", the
-// one the rest of the library is compiled for.
-__device__ __forceinline__ void keep_denorms() { __builtin_amdgcn_s_setreg(1 | (4 << 6) | (1 << 11), 3); }
-__device__ __forceinline__ void flush_denorms() { __builtin_amdgcn_s_setreg(1 | (4 << 6) | (1 << 11), 0); }
-template <class T>
-__device__ __forceinline__ void tie(T& x) {
-  asm volatile("" : "+v"(x));
-}
-// ftz in a flush region (a maximum flushes its operands)
-__device__ __forceinline__ void flush_in_place(float& x) { asm volatile("v_max_f32 %0, %0, %0" : "+v"(x)); }
-
 __device__ __forceinline__ v16f splat(float x) {
   v16f v;
 #pragma unroll

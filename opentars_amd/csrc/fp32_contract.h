@@ -48,6 +48,20 @@ __device__ __forceinline__ float fadd_chain(float acc, float p) {
 }
 __device__ __forceinline__ float chain_end(float acc) { return canon(acc); }
 
+// fp32 subnormals kept / flushed by the hardware (MODE bits 4-5) from here on. In a flush region a plain
+// add is the contract's fadd (it takes ftz of both operands and flushes its sum) up to NaN payloads. The
+// values an instruction of a region takes or gives pass through tie() inside it: the compiler keeps
+// volatile statements in order, so it cannot move the instruction out of its region. Between a kernel's
+// phases the mode is "keep", the one the library is compiled for.
+__device__ __forceinline__ void keep_denorms() { __builtin_amdgcn_s_setreg(1 | (4 << 6) | (1 << 11), 3); }
+__device__ __forceinline__ void flush_denorms() { __builtin_amdgcn_s_setreg(1 | (4 << 6) | (1 << 11), 0); }
+template <class T>
+__device__ __forceinline__ void tie(T& x) {
+  asm volatile("" : "+v"(x));
+}
+// ftz in a flush region (a maximum flushes its operands)
+__device__ __forceinline__ void flush_in_place(float& x) { asm volatile("v_max_f32 %0, %0, %0" : "+v"(x)); }
+
 // A chain run with plain rounded operations (no flushes) equals the contract's chain, up to NaN
 // payloads that chain_end canonicalizes, whenever none of its inputs, products and partial sums is
 // subnormal: every flush is then an identity. Such a chain keeps the minimum of sub_key over those

@@ -1098,12 +1098,6 @@ constexpr int kPvStage = 64, kPvProducers = kPvStage / 4 * kAttnSplitCols;
 constexpr int pv_chain_waves(int Q) { return (Q * kAttnSplitCols + 63) / 64; }
 constexpr int pv_threads(int Q) { return kPvProducers + 64 * pv_chain_waves(Q); }
 
-// fp32 subnormals kept / flushed (MODE bits 4-5) from here on; values that cross a switch pass through
-// tie(), which the compiler keeps in order with it.
-__device__ __forceinline__ void keep_denorms() { __builtin_amdgcn_s_setreg(1 | (4 << 6) | (1 << 11), 3); }
-__device__ __forceinline__ void flush_denorms() { __builtin_amdgcn_s_setreg(1 | (4 << 6) | (1 << 11), 0); }
-__device__ __forceinline__ void tie(float& x) { asm volatile("" : "+v"(x)); }
-
 // A workgroup barrier that orders LDS only: V loads stay in flight across it.
 __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
