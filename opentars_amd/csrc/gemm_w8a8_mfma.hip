@@ -298,7 +298,8 @@ TileTail tile_tail(const MfmaArgs& a) {
   return tl;
 }
 
-// QM_ROWCOL with fp32 output and neither bias nor activation (every K split)
+// QM_ROWCOL with fp32 output and neither bias nor activation (every K split): the general epilogue's code
+// compiled out, as in the GEMV kernels
 bool simple_epilogue(const RowColEpilogue& e) { return e.srow && !e.scol_per_tensor && !e.bias && e.act == 0 && e.out == 0; }
 
 // Stage st of this wave's L blocks into its ring slot (st % S).
@@ -460,22 +461,9 @@ template <int BM, int BN, int WM, int WN, int KS, int S>
 hipError_t go_tile(const MfmaArgs& a, hipStream_t s) {
   static_assert(static_cast<size_t>(S) * (BM + BN) * KS <= 163840, "stage ring exceeds 160 KiB of LDS");
   const int mt = (a.M + BM - 1) / BM, nt = (a.N + BN - 1) / BN;
-  TileTail tl{};
-  for (int i = 0; i < a.nseg; ++i) {
-    tl.W[i] = a.seg[i].W;
-    tl.K[i] = a.seg[i].K;
-    tl.koff[i] = a.seg[i].koff;
-  }
-  tl.nseg = a.nseg;
-  tl.bias = a.epi.bias;
-  tl.scol_per_tensor = a.epi.scol_per_tensor;
-  tl.act = a.epi.act;
-  tl.out = a.epi.out;
-  tl.out_scale = a.epi.out_scale;
-  // QM_ROWCOL with fp32 output and neither bias nor activation (every K split): the general
-  // epilogue's code compiled out, as in the GEMV kernels
+  const TileTail tl = tile_tail(a);
   const RowColEpilogue& e = a.epi;
-  const bool simple = e.srow && !e.scol_per_tensor && !e.bias && e.act == 0 && e.out == 0;
+  const bool simple = simple_epilogue(e);
   const int8_t* A = a.A + a.seg[0].koff;
   const int lda = static_cast<int>(a.lda), ldy = static_cast<int>(a.ldy);
   const dim3 grid(mt * nt), block(64 * WM * WN);
@@ -884,15 +872,9 @@ __global__ __launch_bounds__(256) void mfma_panel_kernel(const int8_t* A, const 
 template <int KQ>
 hipError_t go_panel(const MfmaArgs& a, hipStream_t s) {
   const int mt = (a.M + 63) / 64, nt = (a.N + 47) / 48;
-  TileTail tl{};
-  tl.nseg = 1;
-  tl.bias = a.epi.bias;
-  tl.scol_per_tensor = a.epi.scol_per_tensor;
-  tl.act = a.epi.act;
-  tl.out = a.epi.out;
-  tl.out_scale = a.epi.out_scale;
+  const TileTail tl = tile_tail(a);
   const RowColEpilogue& e = a.epi;
-  const bool simple = e.srow && !e.scol_per_tensor && !e.bias && e.act == 0 && e.out == 0;
+  const bool simple = simple_epilogue(e);
   const int lda = static_cast<int>(a.lda), ldy = static_cast<int>(a.ldy);
   const dim3 grid(mt * nt), block(256);
   if (simple)
@@ -1014,20 +996,9 @@ __global__ __launch_bounds__(64 * KW) void mfma_chunk_kernel(const int8_t* A, co
 
 template <int KW, int DB = 2>
 hipError_t go_chunk(const MfmaArgs& a, hipStream_t s) {
-  TileTail tl{};
-  for (int i = 0; i < a.nseg; ++i) {
-    tl.W[i] = a.seg[i].W;
-    tl.K[i] = a.seg[i].K;
-    tl.koff[i] = a.seg[i].koff;
-  }
-  tl.nseg = a.nseg;
-  tl.bias = a.epi.bias;
-  tl.scol_per_tensor = a.epi.scol_per_tensor;
-  tl.act = a.epi.act;
-  tl.out = a.epi.out;
-  tl.out_scale = a.epi.out_scale;
+  const TileTail tl = tile_tail(a);
   const RowColEpilogue& e = a.epi;
-  const bool simple = e.srow && !e.scol_per_tensor && !e.bias && e.act == 0 && e.out == 0;
+  const bool simple = simple_epilogue(e);
   const int lda = static_cast<int>(a.lda), ldy = static_cast<int>(a.ldy);
   const dim3 grid(a.N / 16), block(64 * KW);
   const int8_t* A = a.A + a.seg[0].koff;
