@@ -494,11 +494,17 @@ hipError_t go_tile(const MfmaArgs& a, hipStream_t s) {
 // multiple of 128 ends in a partial stage: its activation chunks past K read 16 zero bytes, its weight
 // chunks past K the row's last chunk (any bytes: they meet the zeros).
 //
+// (The overlap is whole for the MFMAs of (st, 0). Those of (st, 1) follow a join with the last stage's path, on
+// which only operand reads of their own are pending, so the compiler makes the first of them wait until the
+// reads of (st + 1, 0) have landed too.)
+//
 // Measured at M = 2048, K = N = 4096 on 128 x 256 tiles (one per CU): 8 waves of 64 x 64 outputs 41 us (1.68
 // POP/s; 95 us on the 64 x 64 ring tiles); 4 waves of 64 x 128 61 us (their accumulators and two operand
 // sets pass 256 registers and move through the others); the stages through registers and LDS writes
 // instead of direct loads 45 us; with neither loads nor LDS reads in the loop 33 us, where the matrix
-// cores' clock and the epilogue bound it. More ring slots than these changed nothing.
+// cores' clock and the epilogue bound it. More ring slots than these changed nothing. With the epilogue's
+// operands loaded before the stages 38.5 -> 36.9 us a call (the matrix cores' 32768 busy cycles per SIMD are
+// 13.7 us of it).
 __device__ const int4 kZeroChunk = {0, 0, 0, 0};
 
 template <int BM, int BN, int WM, int WN, int S, bool SIMPLE, bool KSPLIT>
@@ -1029,7 +1035,7 @@ hipError_t go_chunk(const MfmaArgs& a, hipStream_t s) {
 // cold; the results are the same bits for every tile.
 //  * 128 x 256 wide tiles (8 waves) from 192 of them when the last round of 256 is at least 4/5 full (3/4
 //    from K = 2048, where a tile's fill matters less): M = 2048, K = 4096, N = 4096 95 -> 41 us (64 x 64 ring
-//    tiles before; 64 x 128 wide 51 us), M = 3000, K = 1024, N = 3072 (288 tiles: 56%) 33 us against 27 on the next;
+//    tiles before; 64 x 128 wide 51 us; 37 us with the epilogue's operands loaded ahead), M = 3000, K = 1024, N = 3072 (288 tiles: 56%) 33 us against 27 on the next;
 //  * with K blocks of whole 256-byte stages: the 64 x 48 tiles at 192 to 256 of them (in the panel form with one
 //    K block of at most 1280): M = 256, K = 1024, N = 3072 5.0 us (64 x 64 wide 5.7; a second round for a few
 //    tiles is what they lose by: M = 260 7.5 against 5.6); the 32 x 32 ring with 512-byte stages at most 256 of
@@ -1038,8 +1044,9 @@ hipError_t go_chunk(const MfmaArgs& a, hipStream_t s) {
 //    43 -> 24 us, M = 512, K = 1152, N = 6912 35.6 -> 12.0 us (32 x 32 direct tiles before). With GELU and the
 //    activations after it the epilogue weighs as much as the sums, and below 512 tiles a CU with two of them
 //    holds the others up: M = 333, K = 1152, N = 6912 26.6 us, 20.8 us on 64 x 64 wide tiles;
-//  * whole 256-byte stages and at most 512 32 x 32 tiles: the 32 x 32 ring with 256-byte stages (M = 512,
-//    K = 3072, N = 1024 8.2 us, 32 x 64 wide 8.6; at 640 tiles, M = 130, K = N = 4096, 19.6 against 12.0);
+//  * whole 256-byte stages and at most 768 32 x 32 tiles: the 32 x 32 ring with 256-byte stages (M = 512,
+//    K = 3072, N = 1024 8.2 us, 32 x 64 wide 8.6; at 640 tiles, M = 130, K = N = 4096 12.2 us, 64 x 64 wide 12.9; at 768,
+//    M = 72, K = 1024, N = 8192 5.7 and 6.0);
 //  * 64 x 64 wide tiles from 192 of them (M = 777, K = 3072, N = 1024 16.9 -> 10.4 us), else 32 x 64 wide tiles
 //    (M = 64, K = 1152, N = 6912 9.0 -> 5.3 us);
 //  * the direct kernel's 32 x 32 tiles with 4 waves over K for few tiles of a long K that is not whole
@@ -1047,17 +1054,18 @@ hipError_t go_chunk(const MfmaArgs& a, hipStream_t s) {
 //    offsets do not cover. A K split runs the same rules without the 128 x 256 tiles.
 // A general epilogue (anything but fp32 output with row and column scales alone) costs a wave its instructions per
 // output: a 32 x 64 tile gives each of its four waves twice the outputs of a 32 x 32 tile, while SIMDs of a small grid
-// idle. "Chains" are GELU, SILU, sigmoid and softplus, 70 to 120 dependent instructions each. Measured over 1582
-// shapes (M = 17 - 2048, K = 128 - 6912, N = 512 - 12288) with up to seven epilogues each, the lines where the two sides
+// idle. "Chains" are GELU, SILU, sigmoid and softplus, 90 to 220 vector instructions per output. Measured over 1188
+// shapes (M = 17 - 2048, K = 128 - 6912, N = 512 - 12288) with five or seven epilogues each, the lines where the two sides
 // were equal:
 //  * K below 640 and not whole 256-byte stages: the direct 32 x 32 tiles up to 768 of them, with chains up to 1536, with
 //    softplus at any number (M = 64, K = 272, N = 1040, GELU 5.8 us, 32 x 64 wide 7.5; M = 900, K = 272, N = 6912, softplus
 //    45 us, 128 x 256 wide 60; at K = 640 the two are equal at 256 tiles);
 //  * no 128 x 256 tiles with chains below K = 1024, where a CU's one tile ends in 64 outputs per thread with nothing
 //    beside it (M = 900, K = 272, N = 6912, GELU 46 us, 64 x 128 wide 38);
-//  * whole 256-byte stages: the 32 x 32 ring up to 768 tiles (M = 130, K = 1024, N = 4096, INT8 output 6.2 us, 64 x 64 wide
-//    6.7, GELU 8.4 and 10.1), with chains and K up to 2048 again from 257 64 x 64 tiles, the second round of which nearly
-//    every CU would wait for, to 1536 32 x 32 tiles (M = 333, K = 1024, N = 3072, GELU 12.7 us, 64 x 64 wide 14.0);
+//  * whole 256-byte stages: the 32 x 32 ring up to its 768 tiles gains more (M = 130, K = 1024, N = 4096, INT8 output 6.2 us,
+//    64 x 64 wide 6.7, GELU 8.4 and 10.1); with chains and K up to 2048 it is the faster one again from 257 64 x 64 tiles,
+//    where the 256 CUs wait for a few second tiles, to 1536 of its own (M = 333, K = 1024, N = 3072, GELU 12.7 us, 64 x 64
+//    wide 14.0);
 //  * chains on at most 256 32 x 32 tiles of other K: the direct kernel (M = 100, K = 2064, N = 2048, softplus 10.6 us, 32 x 64
 //    wide 12.3).
 bool whole_stages(const MfmaArgs& a, int ks) {
@@ -1106,11 +1114,10 @@ hipError_t run(const MfmaArgs& a, hipStream_t s) {
     return go_tile<64, 48, 4, 1, 256, 3>(a, s);
   }
   if (t32 <= 256 && whole_stages(a, 1024)) return go_tile<32, 32, 2, 2, 512, 3>(a, s);
-  if (whole && !simple && (t32 <= 768 || (chains && t64 > 256 && t32 <= 1536 && longest <= 2048)))
+  if (whole && (t32 <= 768 || (chains && t64 > 256 && t32 <= 1536 && longest <= 2048)))
     return go_tile<32, 32, 2, 2, 256, 3>(a, s);
   if (!whole && chains && t32 <= 256) return go_direct<2, 2, 4, 1>(a, s);
   if (tc >= 192 && (tc >= 512 || a.epi.act < 3)) return go_wide<64, 128, 2, 4, 3>(a, s);
-  if (whole && t32 <= 512) return go_tile<32, 32, 2, 2, 256, 3>(a, s);
   if (t64 >= 192) return go_wide<64, 64, 2, 4, 4>(a, s);
   if (tiles(a, 32, 64) < 96 && longest > 1280) return go_direct<2, 2, 4, 1>(a, s);
   return go_wide<32, 64, 2, 2, 4>(a, s);

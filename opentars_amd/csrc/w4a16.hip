@@ -944,11 +944,12 @@ hipError_t go_cpl(const W4Args& a, int cpl, hipStream_t s) {
 //     weight tiles) with the largest grid of at most 256 workgroups: K = 6144, N = 1536: M = 8 /
 //     16 / 32: 6.6 / 7.8 / 11.6 us; K = 3072, N = 4096: M = 8 / 16: 6.0 / 8.5 us.
 //     The largest grids of both are bound by the waves in flight, which LDS (operands and terms sized for
-//     GMAX groups) limits: with GMAX for the row's groups instead of 16 or 48 (us, M x K x N): up to 4 groups
-//     8 weight tiles of one wave (1000 x 512 x 4096 91 -> 34; 4 tiles 38), up to 8 groups 4 tiles of two
-//     (512 x 1024 x 4096 61 -> 33; at 6 groups 163 -> 87), up to 12 groups 8 tiles of two waves (256 x 1536 x
-//     12288 97 -> 73; 4 tiles 74.5; with GMAX 16 they took 105), 18 to 24 groups two tiles of 8 waves (200 x
-//     3072 x 4096 85 -> 46; one tile of 16 waves 65).
+//     GMAX groups) limits: with GMAX for the row's groups instead of 16 or 48 (us, M x K x N, bf16 rows, weights
+//     cold): up to 4 groups 8 weight tiles of one wave (1000 x 512 x 4096 93 -> 39; 4 tiles 44), up to 8 groups 4
+//     tiles of two (512 x 1024 x 4096 63 -> 36; at 6 groups 56 -> 32), up to 12 groups 8 tiles of two waves (256 x
+//     1536 x 12288 101 -> 70; 4 tiles of two 73, of four 81; 8 with GMAX 16 106) but from 257 to 320 workgroups
+//     (256 CUs: a second round for a few), where 4 tiles with GMAX 16 stay (256 x 1536 x 1280 15.7, 8 tiles 17.6),
+//     18 to 24 groups two tiles of 8 waves (200 x 3072 x 4096 95 -> 53; one tile of 16 waves 74).
 // The 8-row tiles with the two halves of the mantissa in the operand rows replaced tiles that
 // took them in separate MFMAs (4 rows per tile and masked operand rows): K = 1536, N = 12288:
 // M = 4 / 8 / 16 / 32: 6.3 / 9.1 / 12.5 / 22.1 -> 5.7 / 6.7 / 9.9 / 16.6 us.

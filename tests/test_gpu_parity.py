@@ -666,7 +666,8 @@ def test_wide_tiles_with_every_activation(act, out):
     (97, 4112, 656, ACT_SILU, OUT_INT8, "rowcol", True),
     (130, 1040, 272, ACT_SOFTPLUS, OUT_INT8, "rowcol", True), (200, 4112, 528, ACT_GELU, OUT_FP32, "rowcol", False),
     (260, 5648, 16, ACT_SOFTPLUS, OUT_BF16, "tensor", True), (65, 1040, 1040, ACT_SIGMOID, OUT_FP32, "channel", True),
-    (130, 4112, 768, ACT_NONE, OUT_INT8, "rowcol", False), (333, 3088, 512, ACT_GELU, OUT_BF16, "rowcol", True),
+    (130, 4112, 768, ACT_NONE, OUT_INT8, "rowcol", False), (131, 4096, 256, ACT_NONE, OUT_FP32, "rowcol", False),
+    (333, 3088, 512, ACT_GELU, OUT_BF16, "rowcol", True),
 ])
 def test_prompt_rows_by_epilogue(M, N, K, act, out, qm, bias):
     rng = np.random.default_rng(M * 3 + K)
