@@ -1050,8 +1050,9 @@ hipError_t go_chunk(const MfmaArgs& a, hipStream_t s) {
 //  * 64 x 64 wide tiles from 192 of them (M = 777, K = 3072, N = 1024 16.9 -> 10.4 us), else 32 x 64 wide tiles
 //    (M = 64, K = 1152, N = 6912 9.0 -> 5.3 us);
 //  * the direct kernel's 32 x 32 tiles with 4 waves over K for few tiles of a long K that is not whole
-//    stages (M = 20, K = 2064, N = 2048 6.2 us, 32 x 64 wide 6.8) and for row strides the LDS kernels' 32-bit
-//    offsets do not cover. A K split runs the same rules without the 128 x 256 tiles.
+//    stages (M = 20, K = 2064, N = 2048 6.2 us, 32 x 64 wide 6.8); for activation rows 16 MiB or more apart, which the
+//    wide tiles' 32-bit offsets do not cover, the ring and panels where they apply (M = 256, K = N = 4096 16.6 us on the
+//    ring, direct 34), else the direct kernel, and that for any longer stride. A K split runs the same rules without the 128 x 256 tiles.
 // A general epilogue (anything but fp32 output with row and column scales alone) costs a wave its instructions per
 // output: a 32 x 64 tile gives each of its four waves twice the outputs of a 32 x 32 tile, while SIMDs of a small grid
 // idle. "Chains" are GELU, SILU, sigmoid and softplus, 90 to 220 vector instructions per output. Measured over 1188
@@ -1087,8 +1088,10 @@ hipError_t run(const MfmaArgs& a, hipStream_t s) {
     }
     return go_direct<1, 1, 8, 1>(a, s);
   }
-  // the LDS kernels take 32-bit offsets inside a tile's rows; the direct kernel any strides
-  if (a.lda >= (1 << 24) || a.ldy > INT32_MAX) return go_direct<2, 2, 4, 1>(a, s);
+  // the LDS kernels take 32-bit row strides, the wide tiles 32-bit offsets inside a tile's rows too; the direct kernel
+  // any strides
+  if (a.lda > INT32_MAX || a.ldy > INT32_MAX) return go_direct<2, 2, 4, 1>(a, s);
+  const bool wide = a.lda < (1 << 24);
   const bool whole = whole_stages(a, 256);
   int longest = 0;
   for (int i = 0; i < a.nseg; ++i) longest = a.seg[i].K > longest ? a.seg[i].K : longest;
@@ -1098,7 +1101,7 @@ hipError_t run(const MfmaArgs& a, hipStream_t s) {
   const bool simple = a.nseg > 1 || simple_epilogue(a.epi);
   const bool chains = a.epi.act >= 3 && a.epi.act <= 6, softplus = a.epi.act == 6;
   if (!whole && !simple && longest < 640 && (softplus || t32 <= (chains ? 1536 : 768))) return go_direct<2, 2, 4, 1>(a, s);
-  if (a.nseg == 1 && tw >= 192 && !(chains && longest < 1024) &&
+  if (wide && a.nseg == 1 && tw >= 192 && !(chains && longest < 1024) &&
       (5 * tw >= 4 * rounds || (a.seg[0].K >= 2048 && 4 * tw >= 3 * rounds)))
     return go_wide<128, 256, 2, 4, 3>(a, s);
   if (whole && t48 >= 192 && t48 <= 256) {
@@ -1116,7 +1119,8 @@ hipError_t run(const MfmaArgs& a, hipStream_t s) {
   if (t32 <= 256 && whole_stages(a, 1024)) return go_tile<32, 32, 2, 2, 512, 3>(a, s);
   if (whole && (t32 <= 768 || (chains && t64 > 256 && t32 <= 1536 && longest <= 2048)))
     return go_tile<32, 32, 2, 2, 256, 3>(a, s);
-  if (!whole && chains && t32 <= 256) return go_direct<2, 2, 4, 1>(a, s);
+  if (!wide && whole) return go_tile<32, 32, 2, 2, 256, 3>(a, s);
+  if (!wide || (!whole && chains && t32 <= 256)) return go_direct<2, 2, 4, 1>(a, s);
   if (tc >= 192 && (tc >= 512 || a.epi.act < 3)) return go_wide<64, 128, 2, 4, 3>(a, s);
   if (t64 >= 192) return go_wide<64, 64, 2, 4, 4>(a, s);
   if (tiles(a, 32, 64) < 96 && longest > 1280) return go_direct<2, 2, 4, 1>(a, s);

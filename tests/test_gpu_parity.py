@@ -684,6 +684,20 @@ def test_prompt_rows_by_epilogue(M, N, K, act, out, qm, bias):
     assert same(host(y), want), mismatch(host(y), want)
 
 
+@pytest.mark.parametrize("M,N,K", [(40, 1040, 256), (40, 12320, 256), (17, 4112, 272)])
+def test_prompt_rows_16_mib_apart(M, N, K):
+    """Activation rows past the wide tiles' 32-bit offsets: the 32 x 32 ring on whole stages, the direct tiles otherwise."""
+    rng = np.random.default_rng(M + K)
+    A = rng.integers(-128, 128, (M, K), dtype=np.int8)
+    W = rng.integers(-128, 128, (N, K), dtype=np.int8)
+    sc, srow = rng.uniform(1e-4, 3e-2, N).astype(f32), rng.uniform(0.1, 2.0, M).astype(f32)
+    far = torch.empty(((M - 1) << 24) + K, dtype=torch.int8, device="cuda").as_strided((M, K), (1 << 24, 1))
+    far.copy_(torch.from_numpy(A))
+    y = ops.gemm_rowcol(far, cuda(srow), cuda(W), cuda(sc))
+    want = G.gemm_rowcol(A, srow, W, sc)
+    assert same(host(y), want), mismatch(host(y), want)
+
+
 @pytest.mark.parametrize("M,N,blocks", [(100, 12304, [128, 144, 16]), (200, 6160, [512, 256]), (130, 4112, [48, 1040]),
                                         (40, 1040, [272, 128])])
 def test_ksplit_wide_tiles(M, N, blocks):
