@@ -269,9 +269,10 @@ int tars_fdot(const float* A, int64_t lda, const void* B, int64_t ldb, int32_t n
  * of the call's stream, which the library allocates at the stream's first use on the device and
  * keeps until the process ends (each stream has its own, up to 64 streams per device, so calls on
  * different streams may overlap in time; a graph captured from a stream keeps that stream's
- * scratch, so replay it ordered with the stream's other attention calls); otherwise (more streams,
- * or a stream capturing a graph before its first use), one workgroup per head. The bits are the
- * same.
+ * scratch, so replay it ordered with the stream's other attention calls). Two and more rows that
+ * do not fit, or have no scratch (more streams, or a stream capturing a graph before its first
+ * use), run 16 (8 past 2544 keys) query rows of a head per workgroup; one row without a scratch,
+ * and any rows with V rows 128 MiB or more apart, one workgroup per head. The bits are the same.
  */
 int tars_attention(const float* const* q, int64_t ldq, const float* const* k, int64_t ldk,
                    const void* const* v, int64_t ldv, int32_t v_fp16, void* const* att, int64_t ldatt,

@@ -342,8 +342,9 @@ struct AttnArgs {
   int heads, M, nk, hd, causal_k, v_fp16, out;
   float out_scale;
   // The split form (two launches over many workgroups) when scratch is not null and the shape fits
-  // (attention_split_fits); otherwise one workgroup per head. scratch: device memory of
-  // scratch_floats floats holding the scores of every head and query row between the launches.
+  // (attention_split_fits); otherwise prompt rows (launch_attention_rows) or, for one row and for V rows
+  // 128 MiB or more apart, one workgroup per head. scratch: device memory of scratch_floats floats
+  // holding the scores of every head and query row between the launches.
   float* scratch;
   int64_t scratch_floats;
   // set by launch_attention for the split kernels: scratch row stride (floats), query heads per

@@ -735,7 +735,7 @@ tars::AttnNormRope norm_rope_args(uint8_t* image, const Desc& rd, const Desc& pd
   return p;
 }
 
-// scratch: the split form's scores between its two launches (null: one workgroup per head). An
+// scratch: the split form's scores between its two launches (null: the forms without one). An
 // eager dispatch passes its stream's workspace, a launch plan the scratch it owns.
 int launch_attention_group(uint8_t* image, const std::vector<AttnHead>& heads, hipStream_t s, float* scratch,
                            const RopePrologue* pro = nullptr) {

@@ -576,8 +576,9 @@ __global__ __launch_bounds__(256) void fdot_nn_kernel(FdotArgs a) {
 
 // ------------------------------------------------------------------------------ fused decode attention
 // The per-head triple FDOT_NT (scores) -> ROW_SOFTMAX (causal) -> FDOT_NN (P V) of the reference's
-// attention lowering, in two forms with the same bits:
-//  * one workgroup per query head (attn_kernel): (1) the scores s[j] = sum16_k q[k] K[j][k] for
+// attention lowering, in three forms with the same bits. Prompt rows are in attn_rows.hip; here:
+//  * one workgroup per query head (attn_kernel; one row without a scratch, or V rows too far apart for
+//    the prompt-row kernel): (1) the scores s[j] = sum16_k q[k] K[j][k] for
 //    every key (16-lane groups, 16 keys per group (8 at head size 256 or up to 128 keys, 4 up to
 //    64) with their K rows loaded together and their chains interleaved), kept in LDS; (2) the
 //    causal softmax over them in place (as row_lds_kernel); (3) the P V chains over V staged in LDS
@@ -1386,8 +1387,7 @@ float* attention_workspace(hipStream_t s) {
   // One scratch per (device, stream): work on one stream runs in order, so two calls can share a
   // scratch only when they are ordered; calls on different streams get different scratches and
   // may overlap in time. At most kMaxStreams streams per device get one; further streams (and a
-  // stream that is capturing a graph when it would get its first) run the one-workgroup-per-head
-  // form, which needs none.
+  // stream that is capturing a graph when it would get its first) run the forms that need none.
   constexpr int kMaxDevices = 64;
   constexpr size_t kMaxStreams = 64;
   static std::mutex mu;
