@@ -15,8 +15,11 @@
 // range, and by the attention tests' planted values. q, K and V elements are flushed on arrival.
 // NaN payloads are canonicalized where a value is stored; they reach nothing else.
 //
-// A workgroup owns 16 query rows of one head, its scores in LDS. Per (query, key) pair that is 2 hd
-// adds (4 cycles per 64 of them), which bounds the kernel; the MFMAs run beside them.
+// A workgroup owns 16 query rows of one head, its scores in LDS. Per (query, key) pair the contract
+// leaves 2 hd adds (4 cycles of a SIMD per 64 of them): 8208 vector instructions per SIMD for 512 causal
+// rows of 16 heads over 512 keys, 14 us, of the 17915 (30 us) that the kernel issues there in 55 us, next to
+// 16896 busy cycles of the matrix cores (7 us). The rest is the uneven load of the causal tiles, whose
+// workgroups are all resident at once, and a wave left alone on its SIMD at the end.
 //  1. scores, 16 keys per tile, tiles dealt to the waves. Block b of the MFMA takes the chains
 //     4 b + e of sum16 (element 16 u + 4 b + e in step u), e one after another: lane l holds the 16
 //     bytes 64 u + 16 (l / 16) of query row and key row l % 16, so q stays in registers for the
