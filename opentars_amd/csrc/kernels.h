@@ -324,9 +324,10 @@ struct AttnNormRope {
 };
 
 // Elements (keys) row m of a causal softmax over n sees: min(n, causal_k + m), or n when causal_k is 0. A
-// causal_k up to 2^31 - 1 is legal (no mask), so their sum is formed only when it is below n.
+// causal_k up to 2^31 - 1 is legal (no mask): the sum of two such values is below 2^32, so it is formed unsigned.
 __host__ __device__ __forceinline__ int causal_valid(int n, int causal_k, int m) {
-  return causal_k > 0 && m < n - causal_k ? causal_k + m : n;
+  const uint32_t seen = static_cast<uint32_t>(causal_k) + static_cast<uint32_t>(m), all = static_cast<uint32_t>(n);
+  return causal_k > 0 && seen < all ? static_cast<int>(seen) : n;
 }
 
 struct AttnArgs {
