@@ -797,9 +797,10 @@ def test_c5_w4a16_gemma4(K, N, seed):
 
 
 # the largest grids, by groups of a row: 2 to 4, to 8, to 12, to 16, 18 to 24 and more, with a partial last
-# weight tile and a partial last row tile
+# weight tile and a partial last row tile; 10 and 12 groups also on 288 workgroups, which take four weight tiles
 @pytest.mark.parametrize("K,M,N", [(256, 203, 1040), (512, 203, 1040), (768, 203, 1040), (1024, 203, 1040),
                                    (1280, 203, 1040), (1536, 203, 1040), (1792, 203, 1040), (2304, 67, 528),
+                                   (1280, 250, 1040), (1536, 250, 1040),
                                    (3072, 67, 528), (3328, 67, 528)])
 def test_w4a16_large_grids(K, M, N):
     x, Wp, ws, _ = w4_inputs(K + M, M, N, K)
